@@ -215,18 +215,22 @@ __host__ __device__ constexpr int pair_lo(int bits, int q) {
 __host__ __device__ constexpr int pair_hi(int bits, int q) {
   return bits == 2 ? pair_lo(2, q) + 8 : bits == 3 ? pair_lo(3, q) + 16 : bits == 4 ? pair_lo(4, q) + 4 : pair_lo(8, q) + 2;
 }
-// Offset classes: b2 {0,2,4,6,8}, b3 {0,3,6}, b4 {0,4}, b8 {0}.
+// Offset classes: b2 {0,2,4,6,8}, b3 {1,4,7}, b4 {0,4}, b8 {0}.  v_dot2_f32_f16
+// keeps fewer bits of a product the more leading zeros a subnormal factor has,
+// so 3 bits takes the highest offsets that fit the ten-bit mantissa: at
+// {0,3,6}, the same instruction count, only 94-95 % of cfg4-size outputs were
+// the correctly rounded ones.
 __host__ __device__ constexpr int n_classes(int bits) { return bits == 2 ? 5 : bits == 3 ? 3 : bits == 4 ? 2 : 1; }
 __host__ __device__ constexpr int class_of_off(int bits, int off) {
   return bits == 2 ? off / 2 : bits == 3 ? off / 3 : bits == 4 ? off / 4 : off;
 }
 __host__ __device__ constexpr int off_of_class(int bits, int c) {
-  return bits == 2 ? 2 * c : bits == 3 ? 3 * c : bits == 4 ? 4 * c : c;
+  return bits == 2 ? 2 * c : bits == 3 ? 3 * c + 1 : bits == 4 ? 4 * c : c;
 }
 __host__ __device__ constexpr int pair_off(int bits, int q) {
   return bits == 2 ? ((q & 7) < 5 ? 2 * (q & 7) : 2 * (q & 7) - 6)
-       : bits == 3 ? (q == 2 || q == 4 || q == 11 || q == 13 ? 6
-                      : q == 1 || q == 3 || q == 6 || q == 8 || q == 10 || q == 12 ? 3 : 0)
+       : bits == 3 ? (q == 2 || q == 4 || q == 11 || q == 13 ? 7
+                      : q == 1 || q == 3 || q == 6 || q == 8 || q == 10 || q == 12 ? 4 : 1)
        : bits == 4 ? 4 * (q & 1)
        : 0;
 }
@@ -248,31 +252,31 @@ __device__ __forceinline__ void decode_unit(const uint32_t* w, uint32_t (&b)[16]
     }
   } else if constexpr (BITS == 3) {
     // unit bits [0,16) | [48,64), [16,32) | [64,80), [32,48) | [80,96), and
-    // the four codes that straddle those ranges (5, 10, 21, 26); the middle
-    // and last ranges are shifted so that every code sits at offset 0, 3 or 6
-    // of its half (three offset classes instead of eight: 9 VALU fewer per
-    // unit than decoding them in place)
-    const uint32_t m0 = (w[0] & 0x0000ffffu) | (w[1] & 0xffff0000u), m0s = m0 >> 6;
-    const uint32_t m1 = __builtin_amdgcn_alignbit(w[2], w[0], 18), m1s = __builtin_amdgcn_alignbit(w[2], w[0], 24);
-    const uint32_t m2r = (w[1] & 0x0000ffffu) | (w[2] & 0xffff0000u), m2 = m2r >> 1, m2s = m2r >> 7;
-    b[0] = m0 & 0x00070007u;
-    b[1] = m0 & 0x00380038u;
-    b[2] = m0 & 0x01c001c0u;
-    b[3] = m0s & 0x00380038u;
-    b[4] = m0s & 0x01c001c0u;
-    b[5] = m1 & 0x00070007u;
-    b[6] = m1 & 0x00380038u;
-    b[7] = m1s & 0x00070007u;
-    b[8] = m1s & 0x00380038u;
-    b[9] = m2 & 0x00070007u;
-    b[10] = m2 & 0x00380038u;
-    b[11] = m2 & 0x01c001c0u;
-    b[12] = m2s & 0x00380038u;
-    b[13] = m2s & 0x01c001c0u;
-    const uint32_t d0 = __builtin_amdgcn_perm(__builtin_amdgcn_alignbit(w[2], w[1], 31), w[0] >> 15, 0x05040100u);
-    const uint32_t d1 = __builtin_amdgcn_perm(w[2] >> 14, __builtin_amdgcn_alignbit(w[1], w[0], 30), 0x05040100u);
-    b[14] = d0 & 0x00070007u;
-    b[15] = d1 & 0x00070007u;
+    // the four codes that straddle those ranges (5, 10, 21, 26); the first two
+    // ranges are shifted so that every code sits at offset 1, 4 or 7 of its
+    // half (three offset classes instead of eight: 9 VALU fewer per unit than
+    // decoding them in place)
+    const uint32_t m0r = (w[0] & 0x0000ffffu) | (w[1] & 0xffff0000u), m0 = m0r << 1, m0s = m0r >> 5;
+    const uint32_t m1 = __builtin_amdgcn_alignbit(w[2], w[0], 17), m1s = __builtin_amdgcn_alignbit(w[2], w[0], 23);
+    const uint32_t m2 = (w[1] & 0x0000ffffu) | (w[2] & 0xffff0000u), m2s = m2 >> 6;
+    b[0] = m0 & 0x000e000eu;
+    b[1] = m0 & 0x00700070u;
+    b[2] = m0 & 0x03800380u;
+    b[3] = m0s & 0x00700070u;
+    b[4] = m0s & 0x03800380u;
+    b[5] = m1 & 0x000e000eu;
+    b[6] = m1 & 0x00700070u;
+    b[7] = m1s & 0x000e000eu;
+    b[8] = m1s & 0x00700070u;
+    b[9] = m2 & 0x000e000eu;
+    b[10] = m2 & 0x00700070u;
+    b[11] = m2 & 0x03800380u;
+    b[12] = m2s & 0x00700070u;
+    b[13] = m2s & 0x03800380u;
+    const uint32_t d0 = __builtin_amdgcn_perm(__builtin_amdgcn_alignbit(w[2], w[1], 30), w[0] >> 14, 0x05040100u);
+    const uint32_t d1 = __builtin_amdgcn_perm(w[2] >> 13, __builtin_amdgcn_alignbit(w[1], w[0], 29), 0x05040100u);
+    b[14] = d0 & 0x000e000eu;
+    b[15] = d1 & 0x000e000eu;
   } else if constexpr (BITS == 4) {
 #pragma unroll
     for (int d = 0; d < 4; ++d) {
