@@ -36,7 +36,10 @@ ROCM = Path(os.environ.get("ROCM_PATH", "/opt/rocm"))
 HIPCC = str(ROCM / "bin" / "hipcc")
 ARCH = "gfx950"
 
-HIP_SOURCES = ["lb_rowwise.hip", "lb_marlin.hip", "lb_probe.hip", "lb_noalloc.hip"]
+# (source, object name, extra definitions); the rowwise matrix-core product is
+# compiled once per bit width
+HIP_SOURCES = [(f"{n}.hip", n, []) for n in ("lb_rowwise", "lb_marlin", "lb_probe", "lb_noalloc")]
+HIP_SOURCES += [("lb_rowwise_mm.hip", f"lb_rowwise_mm{b}", [f"-DLB_RW_BITS={b}"]) for b in range(2, 9)]
 HIP_FLAGS = [
     f"--offload-arch={ARCH}",
     "-O3",
@@ -88,11 +91,11 @@ def build_library(verbose: bool = True) -> Path:
     LIB_DIR.mkdir(parents=True, exist_ok=True)
     objs = []
     cmds = []
-    for src in HIP_SOURCES:
-        obj = BUILD / (Path(src).stem + ".o")
+    for src, name, defs in HIP_SOURCES:
+        obj = BUILD / f"{name}.o"
         objs.append(obj)
-        cmds.append([HIPCC, *HIP_FLAGS, "-I", str(ROOT / "include"), "-c", str(CSRC / src), "-o", str(obj)])
-    with ThreadPoolExecutor(max_workers=len(cmds)) as ex:
+        cmds.append([HIPCC, *HIP_FLAGS, *defs, "-I", str(ROOT / "include"), "-c", str(CSRC / src), "-o", str(obj)])
+    with ThreadPoolExecutor(max_workers=min(len(cmds), 8)) as ex:
         list(ex.map(_run, cmds))
     hip_rt = _torch_hip_runtime()
     tmp = LIB.with_suffix(".so.tmp")

@@ -5,23 +5,30 @@
 // qweight is an LSB-first bitstream, code c at bits [c*b, c*b+b); value
 // (code - 2^(b-1)) * scale[r, c / group] (csrc/lowbit_gemv.cu:4-14, 16-70).
 //
-// Fast path (row stride % 4 == 0, group % 32 == 0, 16-byte aligned x): one
-// wave per output row; a lane takes 32-code units, which are exactly `b`
-// dwords, so every load is a dword-aligned vector load.  Codes become exact
-// fp16 (code - z) pairs (1024 + code via the fp16 exponent trick, minus
-// 1024 + z), multiplied into fp32 with v_dot2_f32_f16 against the fp16 x pair,
-// and the unit sum is scaled once in fp32.  The wave reduces with DPP/swizzle.
-// General path (any stride / group size): same wave-per-row mapping reading
-// bytes like the reference's scalar decode.
+// One activation row of whole 32-code units: rowwise_lds_kernel (2, 3, 4, 8
+// bits), rowwise_fast_kernel otherwise.  Batches and ragged rows: the matrix-core
+// product (rowwise_mm.hpp).  rowwise_general_kernel takes the rest (groups that
+// are no multiple of 32 columns), reading bytes like the reference's scalar
+// decode.
+//
+// Fast kernel: one wave per output row; a lane takes 32-code units, which are
+// exactly `b` dwords, so every load is a dword-aligned vector load.  Codes
+// become exact fp16 (code - z) pairs (1024 + code via the fp16 exponent trick,
+// minus 1024 + z), multiplied into fp32 with v_dot2_f32_f16 against the fp16 x
+// pair, and the unit sum is scaled once in fp32.  The wave reduces with
+// DPP/swizzle.
+
+#include <algorithm>
 
 #include "lb_common.hpp"
+#include "rowwise_mm_run.hpp"
 
 namespace lb {
 namespace rowwise {
 
 constexpr int kRowsPerWG = 4;
 constexpr int kThreads = kRowsPerWG * kWave;
-constexpr int kMaxBatchTile = 4;
+constexpr int kMaxBatchTile = 4;  // rows of the batch per workgroup of the general kernel
 
 struct Params {
   const uint8_t* q[2];
@@ -30,8 +37,7 @@ struct Params {
   const uint16_t* x;
   int64_t x_stride;      // halves between x rows
   int64_t rows, packed_cols, scale_cols;
-  int64_t cols, group;
-  int batch;
+  int64_t cols, group, batch;
   int unit_shift;        // LDS kernel: log2(group / 32)
 };
 
@@ -82,92 +88,49 @@ __device__ __forceinline__ float unit_dot(const uint32_t* w, const uint32_t* xw,
   return acc;
 }
 
-// Unit sum for a tail unit (codes past `valid` contribute zero).
-template <int BITS>
-__device__ __forceinline__ float unit_dot_tail(const uint32_t* w, const uint16_t* xrow, int64_t c0, int valid) {
-  float acc = 0.f;
-  constexpr int z = 1 << (BITS - 1);
-#pragma unroll
-  for (int t = 0; t < 32; ++t) {
-    if (t < valid) {
-      const int bit = t * BITS;
-      const int d = bit >> 5, s = bit & 31;
-      uint32_t v = (s + BITS <= 32) ? (w[d] >> s) : __builtin_amdgcn_alignbit(w[d + 1], w[d], s);
-      v &= (1u << BITS) - 1u;
-      acc += (float)((int)v - z) * h2f(xrow[c0 + t]);
-    }
-  }
-  return acc;
-}
-
-template <int BITS, int NW, int BT>
+template <int BITS, int NW>
 __global__ __launch_bounds__(kThreads) void rowwise_fast_kernel(Params p) {
   const int wave = threadIdx.x >> 6;
   const int lane = threadIdx.x & 63;
   const int64_t row = (int64_t)blockIdx.x * kRowsPerWG + wave;
-  const int b0 = blockIdx.y * BT;
   if (row >= p.rows) return;
-  const int64_t units = (p.cols + 31) >> 5;
-  const int64_t full_units = p.cols >> 5;
-  const int64_t row_dwords = p.packed_cols >> 2;
+  const int64_t units = p.cols >> 5;
 
-  float acc[NW][BT];
+  float acc[NW];
 #pragma unroll
-  for (int a = 0; a < NW; ++a)
-#pragma unroll
-    for (int b = 0; b < BT; ++b) acc[a][b] = 0.f;
+  for (int a = 0; a < NW; ++a) acc[a] = 0.f;
 
   for (int64_t u = lane; u < units; u += kWave) {
     const int64_t c0 = u << 5;
     const int grp = (int)(c0 / p.group);
     uint32_t w[NW][BITS + 1];
+    float sc[NW];
 #pragma unroll
     for (int a = 0; a < NW; ++a) {
       const uint32_t* src = reinterpret_cast<const uint32_t*>(p.q[a] + row * p.packed_cols) + u * BITS;
-      if (u < full_units) {
 #pragma unroll
-        for (int d = 0; d < BITS; ++d) w[a][d] = __builtin_nontemporal_load(src + d);
-      } else {
-#pragma unroll
-        for (int d = 0; d < BITS; ++d) w[a][d] = (u * BITS + d < row_dwords) ? src[d] : 0u;
-      }
+      for (int d = 0; d < BITS; ++d) w[a][d] = __builtin_nontemporal_load(src + d);
       w[a][BITS] = 0u;
+      sc[a] = h2f(p.s[a][row * p.scale_cols + grp]);
     }
-    float sc[NW];
+    uint32_t xw[16];
+    const uint4* xs = reinterpret_cast<const uint4*>(p.x + c0);
 #pragma unroll
-    for (int a = 0; a < NW; ++a) sc[a] = h2f(p.s[a][row * p.scale_cols + grp]);
-#pragma unroll
-    for (int b = 0; b < BT; ++b) {
-      if (b0 + b < p.batch) {
-        const uint16_t* xrow = p.x + (int64_t)(b0 + b) * p.x_stride;
-        if (u < full_units) {
-          uint32_t xw[16];
-          const uint4* xs = reinterpret_cast<const uint4*>(xrow + c0);
-#pragma unroll
-          for (int v = 0; v < 4; ++v) {
-            const uint4 t4 = xs[v];
-            xw[4 * v] = t4.x;
-            xw[4 * v + 1] = t4.y;
-            xw[4 * v + 2] = t4.z;
-            xw[4 * v + 3] = t4.w;
-          }
-#pragma unroll
-          for (int a = 0; a < NW; ++a) acc[a][b] += sc[a] * unit_dot<BITS, 0>(w[a], xw, 0.f);
-        } else {
-          const int valid = (int)(p.cols - c0);
-#pragma unroll
-          for (int a = 0; a < NW; ++a) acc[a][b] += sc[a] * unit_dot_tail<BITS>(w[a], xrow, c0, valid);
-        }
-      }
+    for (int v = 0; v < 4; ++v) {
+      const uint4 t4 = xs[v];
+      xw[4 * v] = t4.x;
+      xw[4 * v + 1] = t4.y;
+      xw[4 * v + 2] = t4.z;
+      xw[4 * v + 3] = t4.w;
     }
+#pragma unroll
+    for (int a = 0; a < NW; ++a) acc[a] += sc[a] * unit_dot<BITS, 0>(w[a], xw, 0.f);
   }
 #pragma unroll
-  for (int a = 0; a < NW; ++a)
-#pragma unroll
-    for (int b = 0; b < BT; ++b) {
-      const float v = wave_sum(acc[a][b]);
-      if (lane == 0 && b0 + b < p.batch) p.y[a][(int64_t)(b0 + b) * p.rows + row] = f2h(v);
-    }
+  for (int a = 0; a < NW; ++a) {
+    const float v = wave_sum(acc[a]);
+    if (lane == 0) p.y[a][row] = f2h(v);
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -644,15 +607,18 @@ __global__ void row_dequant_kernel(const uint8_t* __restrict__ q, const uint16_t
 }
 
 template <int NW, int BT>
-int launch_bt(const Params& p, int bits, bool fast, hipStream_t st) {
+int launch_general(const Params& p, int bits, hipStream_t st) {
   dim3 grid((unsigned)((p.rows + kRowsPerWG - 1) / kRowsPerWG), (unsigned)((p.batch + BT - 1) / BT));
-  if (!fast) {
-    hipLaunchKernelGGL((rowwise_general_kernel<NW, BT>), grid, dim3(kThreads), 0, st, p, bits);
-    return lbh::launch_status();
-  }
+  hipLaunchKernelGGL((rowwise_general_kernel<NW, BT>), grid, dim3(kThreads), 0, st, p, bits);
+  return lbh::launch_status();
+}
+
+template <int NW>
+int launch_fast(const Params& p, int bits, hipStream_t st) {
+  dim3 grid((unsigned)((p.rows + kRowsPerWG - 1) / kRowsPerWG));
   switch (bits) {
 #define LB_CASE(B) \
-  case B: hipLaunchKernelGGL((rowwise_fast_kernel<B, NW, BT>), grid, dim3(kThreads), 0, st, p); break;
+  case B: hipLaunchKernelGGL((rowwise_fast_kernel<B, NW>), grid, dim3(kThreads), 0, st, p); break;
     LB_CASE(2) LB_CASE(3) LB_CASE(4) LB_CASE(5) LB_CASE(6) LB_CASE(7) LB_CASE(8)
 #undef LB_CASE
     default: return LB_ERR_ARG;
@@ -747,25 +713,78 @@ int launch_lds(const Params& p, int bits, hipStream_t st) {
   }
 }
 
+// The matrix-core product (rowwise_mm.hpp): any stride and alignment, groups of
+// a multiple of 32 columns or one group for the whole row.  Its operands are
+// addressed with 32-bit offsets, so matrices and batches from 4 GB on go in
+// blocks of rows.  span_mul = ceil(2^32 / d) gives t / d exactly while t * d
+// stays below 2^32 (t * (span_mul * d - 2^32) < 2^32).
+bool mm_takes(const Params& p) {
+  if (p.packed_cols >= (int64_t(1) << 31) || p.scale_cols >= (int64_t(1) << 30) || p.x_stride >= (int64_t(1) << 30))
+    return false;
+  return p.group >= p.cols || (p.group % 32 == 0 && (p.cols / 32 + 4) * (p.group / 32) < (int64_t(1) << 32));
+}
+
+int launch_mm(const Params& p, int nw, int bits, hipStream_t st) {
+  constexpr int64_t kSpan = (int64_t(1) << 32) - 1;
+  const int64_t row_step = std::min<int64_t>(std::min<int64_t>(p.rows, 1 << 30), std::max<int64_t>(1, std::min(kSpan / p.packed_cols, kSpan / (2 * p.scale_cols))));
+  const int64_t batch_step = std::min<int64_t>(p.batch, std::max<int64_t>(1, kSpan / (2 * p.x_stride)));
+  const int sps = p.group >= p.cols || p.group % 128 == 0 ? 1 : p.group % 64 == 0 ? 2 : 4;
+  rwmm::Params m{};
+  m.x_stride = p.x_stride; m.y_stride = p.rows; m.packed_cols = p.packed_cols; m.scale_cols = p.scale_cols;
+  m.cols = (int)p.cols;
+  const int64_t d = p.group / (128 / sps);  // scale spans per group
+  m.span_mul = p.group >= p.cols ? 1u : d == 1 ? 0u : (uint32_t)(((int64_t(1) << 32) + d - 1) / d);
+  for (int64_t r = 0; r < p.rows; r += row_step)
+    for (int64_t b = 0; b < p.batch; b += batch_step) {
+      for (int a = 0; a < 2; ++a) {
+        m.q[a] = p.q[a] + r * p.packed_cols;
+        m.s[a] = p.s[a] + r * p.scale_cols;
+        m.y[a] = p.y[a] + b * p.rows + r;
+      }
+      m.x = p.x + b * p.x_stride;
+      m.rows = (int)std::min(row_step, p.rows - r);
+      m.batch = (int)std::min(batch_step, p.batch - b);
+      int e = LB_ERR_ARG;
+      switch (bits) {
+        case 2: e = rwmm::launch<2>(m, sps, nw, st); break;
+        case 3: e = rwmm::launch<3>(m, sps, nw, st); break;
+        case 4: e = rwmm::launch<4>(m, sps, nw, st); break;
+        case 5: e = rwmm::launch<5>(m, sps, nw, st); break;
+        case 6: e = rwmm::launch<6>(m, sps, nw, st); break;
+        case 7: e = rwmm::launch<7>(m, sps, nw, st); break;
+        case 8: e = rwmm::launch<8>(m, sps, nw, st); break;
+      }
+      if (e != LB_OK) return e;
+    }
+  return LB_OK;
+}
+
+// Whole 32-code units of one activation row: the LDS-staged kernel, or the fast
+// kernel at the widths and sizes that one does not take (5, 6, 7 bits at K =
+// 5120, N = 17408: 22.3 / 23.6 / 25.8 us, the matrix-core product 23.1 / 23.0 /
+// 27.7).  Everything else goes to the matrix-core product (ragged rows at that
+// size, 4 bits: 32.6 us against the general kernel's 132; a batch of 16 rows 26
+// against 196 us on four-row tiles of the fast kernel), except groups that
+// are neither a multiple of 32 columns nor the whole row: the general kernel.
 int launch(Params p, int nw, int bits, hipStream_t st) {
-  const bool fast = (p.packed_cols % 4 == 0) && lbh::aligned(p.q[0], 4) && (nw == 1 || lbh::aligned(p.q[1], 4)) &&
-                    (p.group % 32 == 0) && (p.x_stride % 8 == 0) && lbh::aligned(p.x, 16);
-  // one activation row, whole units, staged in LDS
+  const bool units = p.batch == 1 && p.cols % 32 == 0 && (p.packed_cols % 4 == 0) && lbh::aligned(p.q[0], 4) &&
+                     (nw == 1 || lbh::aligned(p.q[1], 4)) && (p.group % 32 == 0) && lbh::aligned(p.x, 16);
+  // staged in LDS
   const int64_t gu = p.group / 32;  // units per group
-  const bool lds = fast && p.batch == 1 && p.cols % 32 == 0 && (bits == 2 || bits == 3 || bits == 4 || bits == 8) &&
+  const bool lds = units && (bits == 2 || bits == 3 || bits == 4 || bits == 8) &&
                    (p.cols >> 5) * kLdsUnitBytes <= kLdsMaxBytes && (gu & (gu - 1)) == 0 &&
                    p.packed_cols * (p.rows > 0 ? 1 : 0) <= (int64_t)0xffffffff / 2 &&
                    p.rows < (int64_t(1) << 31) && p.scale_cols < (int64_t(1) << 31);  // int kernel arguments
   if (lds) {
     p.unit_shift = 0;
     while ((int64_t(1) << p.unit_shift) < gu) ++p.unit_shift;
+    return nw == 1 ? launch_lds<1>(p, bits, st) : launch_lds<2>(p, bits, st);
   }
-  if (lds) return nw == 1 ? launch_lds<1>(p, bits, st) : launch_lds<2>(p, bits, st);
-  if (p.batch <= 1) {
-    return nw == 1 ? launch_bt<1, 1>(p, bits, fast, st) : launch_bt<2, 1>(p, bits, fast, st);
-  }
-  if (p.batch == 2) return nw == 1 ? launch_bt<1, 2>(p, bits, fast, st) : launch_bt<2, 2>(p, bits, fast, st);
-  return nw == 1 ? launch_bt<1, kMaxBatchTile>(p, bits, fast, st) : launch_bt<2, kMaxBatchTile>(p, bits, fast, st);
+  if (units) return nw == 1 ? launch_fast<1>(p, bits, st) : launch_fast<2>(p, bits, st);
+  if (mm_takes(p)) return launch_mm(p, nw, bits, st);
+  if (p.batch <= 1) return nw == 1 ? launch_general<1, 1>(p, bits, st) : launch_general<2, 1>(p, bits, st);
+  if (p.batch == 2) return launch_general<1, 2>(p, bits, st);
+  return launch_general<1, kMaxBatchTile>(p, bits, st);
 }
 
 // Argument checks shared by the rowwise entry points; mirrors check_lowbit_args
@@ -839,7 +858,7 @@ extern "C" int lb_lowbit_gemm(const uint8_t* qweight, int64_t rows, int64_t pack
   p.q[0] = qweight; p.s[0] = scales; p.y[0] = y;
   p.q[1] = qweight; p.s[1] = scales; p.y[1] = y;
   p.x = x; p.x_stride = x_stride; p.rows = rows; p.packed_cols = packed_cols; p.scale_cols = scale_cols;
-  p.cols = cols; p.group = group_size; p.batch = (int)batch;
+  p.cols = cols; p.group = group_size; p.batch = batch;
   return rowwise::launch(p, 1, (int)bits, (hipStream_t)stream);
 }
 

@@ -1,0 +1,73 @@
+// Launches the rowwise matrix-core product at one bit width, LB_RW_BITS (a
+// compile definition: the build compiles this file once per width).
+
+#include <algorithm>
+
+#include "rowwise_mm.hpp"
+
+namespace lb {
+namespace rwmm {
+namespace {
+
+template <int SPS, int MB, int NB, int W, int DEPTH>
+int launch_skinny(const Params& p, int mats, hipStream_t st) {
+  const dim3 grid((unsigned)((p.rows + 16 * NB - 1) / (16 * NB)), (unsigned)((p.batch + 16 * MB - 1) / (16 * MB)),
+                  (unsigned)mats);
+  hipLaunchKernelGGL((skinny_kernel<LB_RW_BITS, SPS, MB, NB, W, DEPTH>), grid, dim3(W * kWave), 0, st, p);
+  return lbh::launch_status();
+}
+
+template <int SPS, int MB, int NB, int DEPTH>
+int launch_tile(const Params& p, hipStream_t st) {
+  const dim3 grid((unsigned)((p.rows + 64 * NB - 1) / (64 * NB)), (unsigned)((p.batch + 16 * MB - 1) / (16 * MB)));
+  hipLaunchKernelGGL((tile_kernel<LB_RW_BITS, SPS, MB, NB, DEPTH, 2>), grid, dim3(kTileThreads), 0, st, p);
+  return lbh::launch_status();
+}
+
+// Which form, from sweeps at 2, 3, 4 and 8 bits over M = 2..384, K x N = 5120 x
+// 17408 and 17408 x 5120 (times below: 4 bits, g128):
+//   up to 16 rows: 32 output rows per workgroup (M = 16: 25 us at N = 5120,
+//     16 rows 35 us, 64 rows 39 us), 16 where that leaves half the CUs idle;
+//   17 to 32: two blocks of 16 (M = 32, N = 5120: 31 us, one block 46);
+//   above, where 64-column tiles of 64 rows do not give every CU one (N = 5120
+//     up to M = 192): four blocks of 16, the waves splitting K (M = 128: 72 us
+//     against 88 us); eight waves where that is one round of workgroups (M =
+//     64: 53 us against 62 us), four otherwise (M = 128: 72 against 89);
+//   else the largest tile that gives 1.5 workgroups per CU (N = 17408: M = 384
+//     102 us on 64 x 256, M = 256 79 us on 64 x 128 against 99, M = 128 51 us on
+//     32 x 128 against 56).
+template <int SPS>
+int launch_sps(const Params& p, int mats, hipStream_t st) {
+  const int64_t cus = lbh::device_cus();
+  auto wgs = [&](int mb, int rows) {
+    return (int64_t)((p.batch + 16 * mb - 1) / (16 * mb)) * ((p.rows + rows - 1) / rows) * mats;
+  };
+  if (p.batch <= 16) {
+    if (2 * wgs(1, 32) >= cus) return launch_skinny<SPS, 1, 2, 8, 2>(p, mats, st);
+    return launch_skinny<SPS, 1, 1, 8, 2>(p, mats, st);
+  }
+  const bool narrow = wgs(4, 64) < cus;
+  if (p.batch <= 32 || narrow) {
+    if (p.batch > 32 && 2 * wgs(4, 32) >= cus) {
+      if (LB_RW_BITS <= 5 && wgs(4, 32) <= cus) return launch_skinny<SPS, 4, 2, LB_RW_BITS <= 5 ? 8 : 4, 1>(p, mats, st);
+      return launch_skinny<SPS, 4, 2, 4, 1>(p, mats, st);
+    }
+    if (2 * wgs(2, 32) >= cus) return launch_skinny<SPS, 2, 2, 8, 1>(p, mats, st);
+    if (2 * wgs(2, 16) >= cus) return launch_skinny<SPS, 2, 1, 8, 1>(p, mats, st);
+    return launch_skinny<SPS, 1, 1, 8, 2>(p, mats, st);
+  }
+  if (2 * wgs(4, 256) >= 3 * cus) return launch_tile<SPS, 4, 4, 1>(p, st);
+  if (2 * wgs(4, 128) >= 3 * cus) return launch_tile<SPS, 4, 2, 1>(p, st);
+  if (p.batch <= 128) return launch_tile<SPS, 2, 2, 2>(p, st);
+  return launch_tile<SPS, 4, 1, 2>(p, st);
+}
+
+}  // namespace
+
+template <>
+int launch<LB_RW_BITS>(const Params& p, int sps, int mats, hipStream_t st) {
+  return sps == 1 ? launch_sps<1>(p, mats, st) : sps == 2 ? launch_sps<2>(p, mats, st) : launch_sps<4>(p, mats, st);
+}
+
+}  // namespace rwmm
+}  // namespace lb
