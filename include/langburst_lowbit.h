@@ -120,7 +120,10 @@ size_t lb_marlin_scratch_bytes(int64_t prob_m, int64_t prob_n, int64_t prob_k, i
  *       tail tiles; stream-K: 1;
  *   [3] decode: 16-row MFMA blocks; split-tail: whole tiles; stream-K: 0;
  *   [4] workgroups; [5] dynamic LDS bytes per workgroup; [6] scratch bytes;
- *   [7] workspace entries used; [8] kernel launches; [9] compute units planned for.
+ *   [7] workspace entries used; [8] kernel launches (form 1 and 2 of variant 1:
+ *   2, the gated activations are formed in a launch of their own; forms 3 and
+ *   4 count the GEMM's alone, variant 1 has that launch before it there too);
+ *   [9] compute units planned for.
  * Returns LB_OK, or the status the entry point would return for the shape. */
 int lb_marlin_describe_plan(int64_t prob_m, int64_t prob_n, int64_t prob_k, int64_t groupsize, int32_t variant,
                             int64_t workspace_len, int64_t* out);
@@ -136,8 +139,8 @@ int lb_marlin_gemm(const uint16_t* A, const int32_t* B, uint16_t* C, const uint1
                    int32_t* workspace, int64_t workspace_len, int64_t groupsize,
                    void* scratch, size_t scratch_bytes, lb_stream_t stream);
 
-/* Same product with A = fp16(silu(mixed[:, :K]) * mixed[:, K:2K]) formed in
- * the kernel; mixed is fp16 [M, 2K].
+/* Same product with A = fp16(silu(mixed[:, :K]) * mixed[:, K:2K]), formed in
+ * the kernel or in scratch first; mixed is fp16 [M, 2K].
  * Replaces marlin_cuda_silu_packed (csrc/marlin_cuda_kernel.cu:1102-1184) as
  * called by lowbit_marlin_gemm_silu_packed_out (csrc/langburst_ext.cpp:131-185). */
 int lb_marlin_gemm_silu_packed(const uint16_t* mixed, const int32_t* B, uint16_t* C, const uint16_t* s,

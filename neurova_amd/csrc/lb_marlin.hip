@@ -174,7 +174,7 @@ struct Plan {
   size_t x_bytes = 0; // decode kernel: staged activations
   size_t partial_bytes = 0;
   size_t keys_bytes = 0;
-  size_t act_bytes = 0;  // A_DIRECT with SiLU-gated A: fp16(silu(g) * u) [M][K], after the partials
+  size_t act_bytes = 0;  // SiLU-gated, A not staged: fp16(silu(g) * u) [M][K], after the partials
 };
 
 constexpr int kSkinnyWGsPerCU = 2;  // decode workgroups resident per CU (register-limited)
@@ -299,7 +299,7 @@ inline Tiling direct_tiling(int64_t m, int64_t n, int64_t k, int64_t workspace_l
   return t;
 }
 
-// `am`: the A mode of the launch (gemm::A_PLAIN or gemm::A_SILU_PACKED);
+// `gated`: the SiLU-gated projection;
 // `argmax`: the fused-argmax variant; `allow_mixed`: the mixed whole-K plan
 // may be used (grouped scales only).
 //
@@ -318,7 +318,7 @@ constexpr int64_t kMixedMaxM = 4;      // rows with the A slice staged (measured
 constexpr int64_t kMixedDirectMaxM = 32;    // rows with A loaded per step, one whole-K tile per CU
 constexpr int64_t kMixedDirectMaxM2 = 8;    // ... and with two whole-K tiles per CU
 
-inline Plan make_plan(int64_t m, int64_t n, int64_t k, int64_t workspace_len, int am, bool argmax = false,
+inline Plan make_plan(int64_t m, int64_t n, int64_t k, int64_t workspace_len, bool gated, bool argmax = false,
                       bool allow_mixed = true) {
   Plan pl;
   pl.n_cg = (int)(n / 256);
@@ -345,7 +345,7 @@ inline Plan make_plan(int64_t m, int64_t n, int64_t k, int64_t workspace_len, in
   const int64_t chunks_all = n / 64, cus_all = device_cus();
   const bool mixed_direct = m > kMixedMaxM && m <= kMixedDirectMaxM && chunks_all * 8 >= cus_all * 5 &&
                             (chunks_all < 2 * cus_all || m <= kMixedDirectMaxM2);
-  if ((m <= kMixedMaxM || mixed_direct) && allow_mixed && !argmax && am == gemm::A_PLAIN) {
+  if ((m <= kMixedMaxM || mixed_direct) && allow_mixed && !argmax && !gated) {
     const int64_t chunks = chunks_all, cus = cus_all;
     const int ksub = skinny::kWaves;  // 1-chunk tiles: the four waves share the k range
     // (measured at K <= 5120 and up to CUs / 8 leftover chunks; a longer K or
@@ -385,7 +385,7 @@ inline Plan make_plan(int64_t m, int64_t n, int64_t k, int64_t workspace_len, in
   if (td.cpw > 0) {
     if (m > skinny::kMaxM) direct = td.cpw != 2;
     else if (ts.cpw == 0) direct = true;
-    else if (am == gemm::A_SILU_PACKED && m <= 4) direct = false;
+    else if (gated && m <= 4) direct = false;
     else direct = td.cpw <= 2 || (ts.cpw == td.cpw && ts.s > td.s);
   }
   const Tiling tl = direct ? td : ts;
@@ -406,16 +406,16 @@ inline Plan make_plan(int64_t m, int64_t n, int64_t k, int64_t workspace_len, in
     const size_t ring = (direct && cpw == skinny::kWaves) ? (size_t)(32 * m + 1) * 16 : 0;
     pl.lds = std::max(std::max(stage, tile), ring);
     pl.partial_bytes = pl.splits > 1 ? align_up((size_t)pl.splits * (size_t)m * (size_t)n * 4) : 0;
-    if (direct && am == gemm::A_SILU_PACKED) pl.act_bytes = align_up((size_t)m * (size_t)k * 2);
+    if (direct && gated) pl.act_bytes = align_up((size_t)m * (size_t)k * 2);
   } else {
     pl.skinny = false;
-    // 128-row tiles (two workgroups per CU) where M fills them; the SiLU-gated
-    // variant keeps 64-row tiles (its A staging registers leave no room).
-    pl.mb = (m >= 128 && am == gemm::A_PLAIN) ? 8 : (m > 32 ? 4 : 2);
+    // 128-row tiles (two workgroups per CU) where M fills them.
+    pl.mb = m >= 128 ? 8 : (m > 32 ? 4 : 2);
+    if (gated) pl.act_bytes = align_up((size_t)m * (size_t)k * 2);
     const int64_t bm = 16 * pl.mb;
     pl.n_mb = (int)((m + bm - 1) / bm);
     const int64_t tiles = (int64_t)pl.n_cg * pl.n_mb;
-    const int64_t slots = (int64_t)gemm::wgs_per_cu(pl.mb, am) * device_cus();
+    const int64_t slots = (int64_t)gemm::wgs_per_cu(pl.mb) * device_cus();
     int64_t full = (tiles / slots) * slots;
     int64_t tail = tiles - full;
     int s = tail > 0 ? choose_tail_splits(tail, slots, groups, pl.mb) : 1;
@@ -508,7 +508,7 @@ int run(Variant var, const uint16_t* a, const int32_t* b, uint16_t* c, const uin
   if (m > skinny::kMaxM && (a_bytes >= (1LL << 31) || k * n / 2 >= (1LL << 31))) return LB_ERR_PROB_SHAPE;
   if (k * n / 2 >= (1LL << 32)) return LB_ERR_PROB_SHAPE;
   const bool gated = var == V_SILU || var == V_SILU_DONE;
-  const Plan pl = make_plan(m, n, k, workspace_len, gated ? gemm::A_SILU_PACKED : gemm::A_PLAIN, var == V_ARGMAX,
+  const Plan pl = make_plan(m, n, k, workspace_len, gated, var == V_ARGMAX,
                             grouped != 0);
   if (var == V_SILU_DONE && !pl.skinny) return LB_ERR_ARG;  // decode batches only
   if (workspace_len < counters_needed(pl, var == V_ARGMAX)) return LB_ERR_WORKSPACE;
@@ -520,24 +520,25 @@ int run(Variant var, const uint16_t* a, const int32_t* b, uint16_t* c, const uin
   float* partial = pl.partial_bytes ? reinterpret_cast<float*>(sc) : nullptr;
   uint64_t* keys = var == V_ARGMAX ? reinterpret_cast<uint64_t*>(sc + pl.partial_bytes) : nullptr;
 
+  // The SiLU-gated A of the plans that do not stage it is formed once into
+  // scratch first (the staged variant forms it in every tile).
+  if (var == V_SILU && pl.act_bytes > 0) {
+    uint16_t* act = reinterpret_cast<uint16_t*>(sc + pl.partial_bytes);
+    hipLaunchKernelGGL(skinny::silu_pack_kernel,
+                       dim3((unsigned)((k / 8 + 255) / 256), (unsigned)std::min<int64_t>(m, 65535)), dim3(256), 0, st, a,
+                       act, (int)m, (int)k);
+    a = act;
+  }
+
   if (pl.direct) {
-    // A fragments loaded per step; the SiLU-gated A is formed once into
-    // scratch first (the staged variant forms it in every tile).
-    const uint16_t* av = a;
-    if (var == V_SILU) {
-      uint16_t* act = reinterpret_cast<uint16_t*>(sc + pl.partial_bytes);
-      const int64_t items = m * (k / 8);
-      hipLaunchKernelGGL(skinny::silu_pack_kernel, dim3((unsigned)((items + 255) / 256)), dim3(256), 0, st, a, act,
-                         (int)m, (int)k);
-      av = act;
-    }
+    // A fragments loaded per step
     // (mixed plans: the whole-K tile count rides in the high bits of the split count)
     const int32_t sp = pl.whole > 0 ? (int32_t)((pl.whole << 16) | pl.splits) : pl.splits;
     const dim3 grid = pl.whole > 0 ? dim3((unsigned)(pl.whole + (int64_t)(pl.n_cg - pl.whole) * pl.splits), 1, 1)
                                    : dim3((unsigned)pl.n_cg, (unsigned)pl.splits, 1);
 #define LB_SKD(AMV, GV, CV, MRV)                                                                                  \
   hipLaunchKernelGGL((skinny::marlin_skinny_kernel<AMV, skinny::EPI_STORE, GV, CV, MRV>), grid,                  \
-                     dim3(skinny::kThreads), pl.lds, st, av, reinterpret_cast<const uint32_t*>(b), s, (int)m, (int)n, \
+                     dim3(skinny::kThreads), pl.lds, st, a, reinterpret_cast<const uint32_t*>(b), s, (int)m, (int)n, \
                      (int)k, sp, partial, workspace, c, nullptr, nullptr, nullptr)
 #define LB_SKDG(AMV, CV, MRV)                               \
   do {                                                      \
@@ -597,34 +598,30 @@ int run(Variant var, const uint16_t* a, const int32_t* b, uint16_t* c, const uin
   p.partial_bytes = (uint32_t)pl.partial_bytes;
   p.kp_total = (int)(k / 32); p.n_cg = pl.n_cg; p.n_mb = pl.n_mb;
   dim3 grid((unsigned)pl.wgs, 1, 1);
-#define LB_GM_SK(MBV, AMV, EPV, GV, SKV) \
-  hipLaunchKernelGGL((gemm::marlin_gemm_kernel<MBV, AMV, EPV, GV, SKV>), grid, dim3(gemm::kThreads), 0, st, p)
-#define LB_GM(MBV, AMV, EPV, GV)                                   \
-  do {                                                             \
-    if constexpr (MBV == 8 && AMV == gemm::A_PLAIN) {              \
-      if (pl.sk_wgs > 0) LB_GM_SK(MBV, AMV, EPV, GV, true);        \
-      else LB_GM_SK(MBV, AMV, EPV, GV, false);                     \
-    } else {                                                       \
-      LB_GM_SK(MBV, AMV, EPV, GV, false);                          \
-    }                                                              \
+#define LB_GM_SK(MBV, EPV, GV, SKV) \
+  hipLaunchKernelGGL((gemm::marlin_gemm_kernel<MBV, EPV, GV, SKV>), grid, dim3(gemm::kThreads), 0, st, p)
+#define LB_GM(MBV, EPV, GV)                                  \
+  do {                                                       \
+    if constexpr (MBV == 8) {                                \
+      if (pl.sk_wgs > 0) LB_GM_SK(MBV, EPV, GV, true);       \
+      else LB_GM_SK(MBV, EPV, GV, false);                    \
+    } else {                                                 \
+      LB_GM_SK(MBV, EPV, GV, false);                         \
+    }                                                        \
   } while (0)
-#define LB_GM_G(MBV, AMV, EPV)                      \
-  do {                                              \
-    if (grouped) LB_GM(MBV, AMV, EPV, true);        \
-    else LB_GM(MBV, AMV, EPV, false);               \
+#define LB_GM_G(MBV, EPV)                      \
+  do {                                         \
+    if (grouped) LB_GM(MBV, EPV, true);        \
+    else LB_GM(MBV, EPV, false);               \
   } while (0)
-#define LB_GM_MB(AMV, EPV)                      \
-  do {                                          \
-    if (pl.mb == 8) LB_GM_G(8, AMV, EPV);       \
-    else if (pl.mb == 4) LB_GM_G(4, AMV, EPV);  \
-    else LB_GM_G(2, AMV, EPV);                  \
+#define LB_GM_MB(EPV)                      \
+  do {                                     \
+    if (pl.mb == 8) LB_GM_G(8, EPV);       \
+    else if (pl.mb == 4) LB_GM_G(4, EPV);  \
+    else LB_GM_G(2, EPV);                  \
   } while (0)
-  if (var == V_PLAIN) LB_GM_MB(gemm::A_PLAIN, gemm::EPI_STORE);
-  else if (var == V_SILU) {  // 64-row tiles at most (see make_plan)
-    if (pl.mb == 4) LB_GM_G(4, gemm::A_SILU_PACKED, gemm::EPI_STORE);
-    else LB_GM_G(2, gemm::A_SILU_PACKED, gemm::EPI_STORE);
-  }
-  else LB_GM_MB(gemm::A_PLAIN, gemm::EPI_ARGMAX);
+  if (var == V_ARGMAX) LB_GM_MB(gemm::EPI_ARGMAX);
+  else LB_GM_MB(gemm::EPI_STORE);
 #undef LB_GM_MB
 #undef LB_GM_G
 #undef LB_GM
@@ -658,12 +655,12 @@ extern "C" size_t lb_marlin_scratch_bytes(int64_t prob_m, int64_t prob_n, int64_
   (void)groupsize;
   if (prob_m <= 0 || prob_n <= 0 || prob_k <= 0 || prob_n % 256 || prob_k % 128) return 0;
   // Plan with an unconstrained workspace: the largest scratch any plan uses.
-  // Largest over the variants (the SiLU-gated one may use other tiles).
+  // Largest over the variants (the SiLU-gated one also holds its activations).
   // (with and without the mixed plan, which only grouped scales take)
-  const marlin::Plan a = marlin::make_plan(prob_m, prob_n, prob_k, INT64_MAX, gemm::A_PLAIN);
-  const marlin::Plan a2 = marlin::make_plan(prob_m, prob_n, prob_k, INT64_MAX, gemm::A_PLAIN, false, false);
-  const marlin::Plan b = marlin::make_plan(prob_m, prob_n, prob_k, INT64_MAX, gemm::A_SILU_PACKED);
-  const marlin::Plan c = marlin::make_plan(prob_m, prob_n, prob_k, INT64_MAX, gemm::A_PLAIN, true);
+  const marlin::Plan a = marlin::make_plan(prob_m, prob_n, prob_k, INT64_MAX, false);
+  const marlin::Plan a2 = marlin::make_plan(prob_m, prob_n, prob_k, INT64_MAX, false, false, false);
+  const marlin::Plan b = marlin::make_plan(prob_m, prob_n, prob_k, INT64_MAX, true);
+  const marlin::Plan c = marlin::make_plan(prob_m, prob_n, prob_k, INT64_MAX, false, true);
   return std::max(std::max(std::max(a.partial_bytes + a.keys_bytes, a2.partial_bytes + a2.keys_bytes),
                            b.partial_bytes + b.keys_bytes + b.act_bytes),
                   c.partial_bytes + c.keys_bytes);
@@ -679,7 +676,7 @@ extern "C" int lb_marlin_describe_plan(int64_t prob_m, int64_t prob_n, int64_t p
   if (prob_m == 0 || prob_n == 0 || prob_k == 0) return LB_OK;
   const bool argmax = variant == 2, gated = variant == 1;
   const marlin::Plan pl = marlin::make_plan(prob_m, prob_n, prob_k, workspace_len,
-                                            gated ? gemm::A_SILU_PACKED : gemm::A_PLAIN, argmax, grouped != 0);
+                                            gated, argmax, grouped != 0);
   if (pl.skinny) {
     out[0] = !pl.direct ? 0 : pl.cpw == skinny::kWaves ? 2 : 1;
     out[1] = pl.cpw;
@@ -832,9 +829,9 @@ FusedMlpPlan fused_mlp_plan(int64_t batch, int64_t hidden, int64_t inter, bool g
   // scales), except that from M = 5 the gate/up launch keeps the 2- or 4-chunk
   // tiles that can pair gate and up chunks (its SiLU-gated store saves the
   // down launch's separate gating pass)
-  p.up = marlin::make_plan(batch, 2 * inter, hidden, INT64_MAX, gemm::A_PLAIN, false,
+  p.up = marlin::make_plan(batch, 2 * inter, hidden, INT64_MAX, false, false,
                            g1 && batch <= marlin::kMixedMaxM);
-  p.down = marlin::make_plan(batch, hidden, inter, INT64_MAX, gemm::A_SILU_PACKED, false, g2);
+  p.down = marlin::make_plan(batch, hidden, inter, INT64_MAX, true, false, g2);
   // decode tiles of 2 or 4 chunks pair gate and up chunks; single-chunk tiles
   // and prefill tiles take the [g | u] round trip
   p.act_path = p.up.skinny && p.up.cpw >= 2 && p.down.skinny;

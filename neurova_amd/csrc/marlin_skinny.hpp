@@ -889,20 +889,21 @@ __global__ __launch_bounds__(kThreads) void marlin_skinny_kernel(const uint16_t*
   skinny_tile<AM, EPI, GROUPED, CPW, MR>(p, cg, split);
 }
 
-// SiLU-gated activations for the A_DIRECT launches: act[m][k] =
+// SiLU-gated activations for the launches that do not stage A: act[m][k] =
 // fp16(silu(g) * u) of mixed [M, 2K] = [g | u], with the staging's own
-// function (silu_mul2), so the direct launch sees the values the staged
-// A_SILU_PACKED variant would.  One thread per 8 halves.
+// function (silu_mul2), so they see the values the staged A_SILU_PACKED variant
+// would.  One thread per 8 halves of a row; rows blockIdx.y, + gridDim.y, ...
+// Bound by its 6 bytes per activation (M = 2048, K = 17408: 214 MB).
 __global__ __launch_bounds__(256) void silu_pack_kernel(const uint16_t* __restrict__ mixed, uint16_t* __restrict__ act,
                                                         int m, int k) {
-  const int64_t octs = (int64_t)k >> 3;
-  const int64_t it = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (it >= (int64_t)m * octs) return;
-  const int64_t row = it / octs, o = it - row * octs;
-  const uint4 g = *reinterpret_cast<const uint4*>(mixed + row * 2 * k + 8 * o);
-  const uint4 u = *reinterpret_cast<const uint4*>(mixed + row * 2 * k + k + 8 * o);
-  *reinterpret_cast<uint4*>(act + row * k + 8 * o) =
-      make_uint4(silu_mul2(g.x, u.x), silu_mul2(g.y, u.y), silu_mul2(g.z, u.z), silu_mul2(g.w, u.w));
+  const int k8 = 8 * (int)(blockIdx.x * 256 + threadIdx.x);
+  if (k8 >= k) return;
+  for (int64_t row = blockIdx.y; row < m; row += gridDim.y) {
+    const uint4 g = *reinterpret_cast<const uint4*>(mixed + row * 2 * k + k8);
+    const uint4 u = *reinterpret_cast<const uint4*>(mixed + row * 2 * k + k + k8);
+    *reinterpret_cast<uint4*>(act + row * k + k8) =
+        make_uint4(silu_mul2(g.x, u.x), silu_mul2(g.y, u.y), silu_mul2(g.z, u.z), silu_mul2(g.w, u.w));
+  }
 }
 
 }  // namespace skinny
