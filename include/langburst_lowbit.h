@@ -120,10 +120,11 @@ size_t lb_marlin_scratch_bytes(int64_t prob_m, int64_t prob_n, int64_t prob_k, i
  *       tail tiles; stream-K: 1;
  *   [3] decode: 16-row MFMA blocks; split-tail: whole tiles; stream-K: 0;
  *   [4] workgroups; [5] dynamic LDS bytes per workgroup; [6] scratch bytes;
- *   [7] workspace entries used; [8] kernel launches (form 1 and 2 of variant 1:
+ *   [7] workspace entries used; [8] kernel launches (forms 1 and 2 of variant 1:
  *   2, the gated activations are formed in a launch of their own; forms 3 and
- *   4 count the GEMM's alone, variant 1 has that launch before it there too);
- *   [9] compute units planned for.
+ *   4 count the GEMM's launch alone: variant 1 has that one before it, and a
+ *   form 3 plan with every tile split, [2] > 1 and [3] = 0, one that sums the
+ *   partials after it); [9] compute units planned for.
  * Returns LB_OK, or the status the entry point would return for the shape. */
 int lb_marlin_describe_plan(int64_t prob_m, int64_t prob_n, int64_t prob_k, int64_t groupsize, int32_t variant,
                             int64_t workspace_len, int64_t* out);

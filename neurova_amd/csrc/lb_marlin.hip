@@ -168,6 +168,7 @@ struct Plan {
   int full_tiles = 0;   // GEMM: tiles computed whole
   int tail_tiles = 0;   // GEMM: tiles split over K ...
   int tail_splits = 1;  // ... this many ways
+  bool two_pass = false; // GEMM: every tile is split and a second launch sums the partials
   int sk_wgs = 0;       // GEMM: > 0, the stream-K schedule over this many workgroups
   int64_t wgs = 0;      // GEMM workgroups
   size_t lds = 0;    // decode kernel dynamic LDS
@@ -207,11 +208,58 @@ inline int choose_tail_splits(int64_t tail, int64_t slots, int groups, int mb) {
   return best;
 }
 
+// Tile height and k split where 128-row tiles fill less than one round: the
+// workgroups a CU holds at a time run their stages together, so a launch takes
+//   first loads and epilogue  +  sum over rounds of stages x stage time at that
+//   residency  +  with splits, the reduce launch and the partials' traffic.
+// The stage times (ns, MB = 2, 4, 8 row blocks with 1, 2, 3 workgroups per CU)
+// and the other constants are a least-squares fit to 1500 launches (M = 33 ..
+// 1024, K x N = 1024 x 2048 .. 5120 x 34816 and 17408 x 5120, 1 .. 20 splits; rms error
+// 7 %); the shape it picks is 1.7 % slower than the best one on average, 13 % at
+// most.  Against the fixed heights and splits summed by the last arrival: M = 64,
+// K = 17408, N = 5120 34.5 -> 24.3 us, M = 128, K = N = 5120 36.1 -> 17.8 us, M =
+// 200, N = 7168 37.6 -> 30.1 us.
+struct GemmShape {
+  int mb = 8, splits = 1;
+};
+inline GemmShape choose_gemm_shape(int64_t m, int64_t n_cg, int groups, int64_t cus) {
+  struct Height {
+    int mb, resident;
+    int64_t stage_ns[3];
+  };
+  static const Height heights[] = {{8, 2, {1640, 2700, 0}}, {4, 3, {1130, 1850, 2700}}, {2, 3, {800, 1400, 1900}}};
+  constexpr int64_t kReduceNs = 1500;         // the second launch
+  constexpr int64_t kPartialNsPerBlock = 5;   // 16 KiB of partials (one row block x 256 columns) written and read
+  constexpr int kMaxSplits = 20;
+  GemmShape best;
+  int64_t best_ns = INT64_MAX;
+  for (const Height& h : heights) {
+    if (h.mb == 8 && m <= 64) continue;   // half the rows of a tile padding
+    if (h.mb == 2 && m > 160) continue;   // weights dequantised for 32 rows at a time: never ahead there
+    const int64_t tiles = n_cg * ((m + 16 * h.mb - 1) / (16 * h.mb));
+    for (int s = 1; s <= kMaxSplits && s <= groups; ++s) {
+      const int64_t wgs = tiles * s;
+      if (s > 1 && (wgs > h.resident * cus || (size_t)wgs * 16 * h.mb * gemm::kThreads * 4 >= ((size_t)1 << 31))) break;
+      const int64_t stages = (groups + s - 1) / s;
+      const int64_t full = wgs / (h.resident * cus), rest = wgs % (h.resident * cus);
+      int64_t ns = full * stages * h.stage_ns[h.resident - 1];
+      if (rest > 0) ns += stages * h.stage_ns[(rest + cus - 1) / cus - 1];
+      if (s > 1) ns += kReduceNs + kPartialNsPerBlock * h.mb * wgs;
+      if (ns < best_ns) {
+        best_ns = ns;
+        best.mb = h.mb;
+        best.splits = s;
+      }
+    }
+  }
+  return best;
+}
+
 // Decode tiling with `cpw` chunks per workgroup: the k split count, or 0
 // when the tiling cannot run (some wave would get no scale group, or the
 // staged A slice does not fit LDS without the workspace to split K).
 // `direct`: A is not staged (skinny::A_DIRECT), so LDS sets no bound.
-inline int skinny_splits(int64_t m, int64_t n, int64_t k, int64_t workspace_len, int cpw, bool direct = false) {
+inline int skinny_splits(int64_t m, int64_t n, int64_t k, int64_t workspace_len, int cus, int cpw, bool direct = false) {
   const int n_cg = (int)(n / (64 * cpw));
   const int ksub = skinny::kWaves / cpw;
   const int groups = (int)(k / 128);
@@ -220,7 +268,7 @@ inline int skinny_splits(int64_t m, int64_t n, int64_t k, int64_t workspace_len,
   const bool can_split = workspace_len >= 1 + (cpw == skinny::kWaves ? n / 64 : (int64_t)n_cg);
   // As many k splits as fit in one wave of resident workgroups: a second,
   // partial wave would cost a whole workgroup's time for a few tiles.
-  int s = (kSkinnyWGsPerCU * device_cus()) / n_cg;
+  int s = (kSkinnyWGsPerCU * cus) / n_cg;
   // split-K partials (S * M * N fp32, written once and read once) stay
   // within half the weight bytes (K * N / 2): S * M <= K / 32
   const int s_traffic = (int)std::max<int64_t>(1, k / (32 * m));
@@ -248,10 +296,10 @@ struct Tiling {
 // Staged A (M <= 16): 4 chunks (one per wave) per workgroup, unless the
 // narrow N then needs more than kSkinnyMaxSplits k splits to fill the chip:
 // then 2 or 1 chunks, whose waves share the workgroup's k range.
-inline Tiling staged_tiling(int64_t m, int64_t n, int64_t k, int64_t workspace_len) {
+inline Tiling staged_tiling(int64_t m, int64_t n, int64_t k, int64_t workspace_len, int cus) {
   Tiling t;
   for (int c = skinny::kWaves; c >= 1; c /= 2) {
-    const int sc = skinny_splits(m, n, k, workspace_len, c);
+    const int sc = skinny_splits(m, n, k, workspace_len, cus, c);
     if (sc == 0) continue;
     if (t.cpw == 0 || sc < t.s) {
       t.cpw = c;
@@ -267,7 +315,7 @@ inline Tiling staged_tiling(int64_t m, int64_t n, int64_t k, int64_t workspace_l
 // every CU a workgroup (4-chunk tiles, whose waves share A through the LDS
 // ring) or 1.5 workgroups per CU (narrower tiles, each wave loading its own
 // A), else the one with the most workgroups.
-inline Tiling direct_tiling(int64_t m, int64_t n, int64_t k, int64_t workspace_len) {
+inline Tiling direct_tiling(int64_t m, int64_t n, int64_t k, int64_t workspace_len, int cus) {
   Tiling t;
   // From M = 12 (M = 8 at long K) with fewer 64-column chunks than CUs:
   // single-chunk tiles split to about one workgroup per CU instead of two
@@ -276,9 +324,9 @@ inline Tiling direct_tiling(int64_t m, int64_t n, int64_t k, int64_t workspace_l
   // 9.8 against 10.1; M = 12 even at K = 5120, 14.3 against 15.1 at K = 17408;
   // M = 8: 13.6 against 14.1 at K = 17408, 0.3 us slower at K = 5120, as at M
   // = 1 and 4)
-  if ((m >= 12 || (m >= 8 && k > 8192)) && n / 64 < device_cus() && k / 128 >= skinny::kWaves) {
+  if ((m >= 12 || (m >= 8 && k > 8192)) && n / 64 < cus && k / 128 >= skinny::kWaves) {
     const int64_t tiles = n / 64;
-    int s = (int)std::max<int64_t>(1, device_cus() / tiles);
+    int s = (int)std::max<int64_t>(1, cus / tiles);
     s = std::min<int>(s, (int)std::max<int64_t>(1, k / (32 * m)));  // partials within half the weight bytes
     s = std::min<int>(s, (int)(k / 128 / skinny::kWaves));  // every wave a scale group
     if (workspace_len < 1 + tiles) s = 1;
@@ -286,10 +334,10 @@ inline Tiling direct_tiling(int64_t m, int64_t n, int64_t k, int64_t workspace_l
   }
   int64_t most = -1;
   for (int c = skinny::kWaves; c >= 1; c /= 2) {
-    const int sc = skinny_splits(m, n, k, workspace_len, c, true);
+    const int sc = skinny_splits(m, n, k, workspace_len, cus, c, true);
     if (sc == 0) continue;
     const int64_t w = (n / (64 * c)) * sc;
-    const int64_t fill = c == skinny::kWaves ? device_cus() : 3 * (int64_t)device_cus() / 2;
+    const int64_t fill = c == skinny::kWaves ? cus : 3 * (int64_t)cus / 2;
     if (sc <= kSkinnyMaxSplits && w >= fill) return Tiling{c, sc};
     if (w > most) {
       most = w;
@@ -300,8 +348,8 @@ inline Tiling direct_tiling(int64_t m, int64_t n, int64_t k, int64_t workspace_l
 }
 
 // `gated`: the SiLU-gated projection;
-// `argmax`: the fused-argmax variant; `allow_mixed`: the mixed whole-K plan
-// may be used (grouped scales only).
+// `argmax`: the fused-argmax variant; `grouped`: group scales (else one per
+// column); `allow_mixed`: the mixed whole-K plan (grouped only) may be used.
 //
 // Which decode form (measured on the decode shapes of BASELINE.json): the direct
 // form where the tiles are narrow (the waves of a workgroup then share
@@ -319,7 +367,7 @@ constexpr int64_t kMixedDirectMaxM = 32;    // rows with A loaded per step, one 
 constexpr int64_t kMixedDirectMaxM2 = 8;    // ... and with two whole-K tiles per CU
 
 inline Plan make_plan(int64_t m, int64_t n, int64_t k, int64_t workspace_len, bool gated, bool argmax = false,
-                      bool allow_mixed = true) {
+                      bool grouped = true, bool allow_mixed = true) {
   Plan pl;
   pl.n_cg = (int)(n / 256);
   const int groups = (int)(k / 128);
@@ -342,11 +390,12 @@ inline Plan make_plan(int64_t m, int64_t n, int64_t k, int64_t workspace_len, bo
   // M = 16 11.5 against 12.5; at half, N = 8192, M = 32 18.3 against 14.3) or
   // two per CU up to M = 8 (N = 34816, M = 8: 20.9 against 22.6 us; M = 16 even,
   // M = 32 39.2 against 31.2 on the ring tiles).
-  const int64_t chunks_all = n / 64, cus_all = device_cus();
-  const bool mixed_direct = m > kMixedMaxM && m <= kMixedDirectMaxM && chunks_all * 8 >= cus_all * 5 &&
-                            (chunks_all < 2 * cus_all || m <= kMixedDirectMaxM2);
-  if ((m <= kMixedMaxM || mixed_direct) && allow_mixed && !argmax && !gated) {
-    const int64_t chunks = chunks_all, cus = cus_all;
+  const int cus = device_cus();  // asked for once: it is a call into the runtime
+  const int64_t chunks_all = n / 64;
+  const bool mixed_direct = m > kMixedMaxM && m <= kMixedDirectMaxM && chunks_all * 8 >= cus * 5 &&
+                            (chunks_all < 2 * cus || m <= kMixedDirectMaxM2);
+  if ((m <= kMixedMaxM || mixed_direct) && allow_mixed && grouped && !argmax && !gated) {
+    const int64_t chunks = chunks_all;
     const int ksub = skinny::kWaves;  // 1-chunk tiles: the four waves share the k range
     // (measured at K <= 5120 and up to CUs / 8 leftover chunks; a longer K or
     // more leftover work per CU keeps the split tiles)
@@ -378,8 +427,8 @@ inline Plan make_plan(int64_t m, int64_t n, int64_t k, int64_t workspace_len, bo
       }
     }
   }
-  const Tiling ts = m <= skinny::kMaxM ? staged_tiling(m, n, k, workspace_len) : Tiling{};
-  const Tiling td = (!argmax && m <= 16 * skinny::kMaxMR) ? direct_tiling(m, n, k, workspace_len)
+  const Tiling ts = m <= skinny::kMaxM ? staged_tiling(m, n, k, workspace_len, cus) : Tiling{};
+  const Tiling td = (!argmax && m <= 16 * skinny::kMaxMR) ? direct_tiling(m, n, k, workspace_len, cus)
                                                                          : Tiling{};
   bool direct = false;
   if (td.cpw > 0) {
@@ -409,26 +458,66 @@ inline Plan make_plan(int64_t m, int64_t n, int64_t k, int64_t workspace_len, bo
     if (direct && gated) pl.act_bytes = align_up((size_t)m * (size_t)k * 2);
   } else {
     pl.skinny = false;
-    // 128-row tiles (two workgroups per CU) where M fills them.
-    pl.mb = m >= 128 ? 8 : (m > 32 ? 4 : 2);
     if (gated) pl.act_bytes = align_up((size_t)m * (size_t)k * 2);
+    pl.keys_bytes = align_up((size_t)m * (size_t)pl.n_cg * 8);
+    const int64_t slots = (int64_t)gemm::wgs_per_cu(8) * cus;      // of 128-row tiles
+    const int64_t tiles8 = (int64_t)pl.n_cg * ((m + 127) / 128);
+    if (!argmax && tiles8 < slots) {
+      // Less than one round of 128-row tiles: stream-K where it is ahead, else
+      // the tile height and k split the cost model prefers.
+      //
+      // Stream-K (every slot runs the same number of stages, a tile is cut
+      // only where a workgroup's range ends; two partial slots per workgroup)
+      // from half a round, and of that range only: just above half, where whole
+      // tiles would leave nearly half of the slots idle (264 tiles: K = 5120
+      // 103.6 us against 106.5, K = 17408 267-284 against 285; at K = 1024
+      // whole tiles would be ahead, 28 against 49 us); long K with tile counts
+      // of whole sixty-fours, whose workgroups on one XCD start at the same k
+      // offset (K = 17408: 320 tiles 301 us against 318 for three splits and
+      // 361 whole, but 300 tiles 335 against 300, 392 tiles 424 against 375
+      // whole); and one scale per column with a short K, which was not measured
+      // against the other forms.  Elsewhere whole tiles are ahead by up to a
+      // factor of two (M = 2048, K = 5120: N = 7168, 448 tiles, 124 against
+      // 144 us, N = 5120, 320 tiles, 110 against 118; K = 1024, N = 5120 31
+      // against 60 us).
+      const size_t sk_bytes = (size_t)2 * slots * 16 * 8 * gemm::kThreads * 4;
+      const bool sk = tiles8 * 100 <= slots * 52 || (!grouped && k <= 2048) ||
+                      (k > 8192 && tiles8 % 64 == 0 && tiles8 * 4 <= slots * 3);
+      if (sk && tiles8 * 2 >= slots && workspace_len >= 1 + tiles8 && sk_bytes < ((size_t)1 << 31) &&
+          (int64_t)groups * tiles8 < ((int64_t)1 << 31)) {
+        pl.mb = 8;
+        pl.n_mb = (int)((m + 127) / 128);
+        pl.sk_wgs = (int)slots;
+        pl.full_tiles = 0;
+        pl.tail_tiles = (int)tiles8;
+        pl.tail_splits = 1;
+        pl.wgs = slots;
+        pl.partial_bytes = align_up(sk_bytes);
+        return pl;
+      }
+      const GemmShape g = choose_gemm_shape(m, pl.n_cg, groups, cus);
+      pl.mb = g.mb;
+      pl.n_mb = (int)((m + 16 * g.mb - 1) / (16 * g.mb));
+      const int64_t tiles = (int64_t)pl.n_cg * pl.n_mb;
+      pl.two_pass = g.splits > 1;
+      pl.full_tiles = pl.two_pass ? 0 : (int)tiles;
+      pl.tail_tiles = pl.two_pass ? (int)tiles : 0;
+      pl.tail_splits = g.splits;
+      pl.wgs = tiles * g.splits;
+      pl.partial_bytes = pl.two_pass ? align_up((size_t)tiles * g.splits * 16 * pl.mb * gemm::kThreads * 4) : 0;
+      return pl;
+    }
+    // A round of 128-row tiles or more: they run whole, as many as fill the
+    // resident slots a whole number of times, and the rest is split over K.
+    // (The argmax also takes this path with fewer tiles, 64 rows below M = 128.)
+    pl.mb = m >= 128 ? 8 : (m > 32 ? 4 : 2);
     const int64_t bm = 16 * pl.mb;
     pl.n_mb = (int)((m + bm - 1) / bm);
     const int64_t tiles = (int64_t)pl.n_cg * pl.n_mb;
-    const int64_t slots = (int64_t)gemm::wgs_per_cu(pl.mb) * device_cus();
-    int64_t full = (tiles / slots) * slots;
+    const int64_t slots_mb = (int64_t)gemm::wgs_per_cu(pl.mb) * cus;
+    int64_t full = (tiles / slots_mb) * slots_mb;
     int64_t tail = tiles - full;
-    int s = tail > 0 ? choose_tail_splits(tail, slots, groups, pl.mb) : 1;
-    // Few rows: the kernel streams B and is bound by bandwidth, not by the
-    // MFMAs the cost model above prices; split further so that every CU gets
-    // a workgroup, as long as the fp32 partials (written and read once) stay
-    // within half the weight bytes: S <= K / (32 * tile rows).
-    if (tail > 0 && m <= 64) {
-      const int s_fill = (int)((device_cus() + tail - 1) / tail);
-      const int s_cap = (int)std::max<int64_t>(1, k / (32 * bm));
-      const int s_mem = std::min(std::min(s_fill, s_cap), groups);
-      if (s_mem > s) s = s_mem;
-    }
+    int s = tail > 0 ? choose_tail_splits(tail, slots_mb, groups, pl.mb) : 1;
     if (s > 1 && workspace_len < 1 + tail) s = 1;
     // partials are addressed through a 32-bit buffer resource
     while (s > 1 && (size_t)tail * s * 16 * pl.mb * gemm::kThreads * 4 >= ((size_t)1 << 31)) --s;
@@ -436,33 +525,12 @@ inline Plan make_plan(int64_t m, int64_t n, int64_t k, int64_t workspace_len, bo
       full = tiles;
       tail = 0;
     }
-    // Stream-K where 128-row tiles fill between half of one round of the
-    // resident slots and all of it: every slot then runs the same number of
-    // stages, and a tile is cut only where a workgroup's range ends.  M = 2048,
-    // K = 17408, N = 5120 (320 tiles on 512 slots): 310 us against 321 us for
-    // 960 third-tiles (1.875 rounds).  With a full round or more the split tail
-    // stays ahead (K = 5120, N = 17408, 1088 tiles: 299 us against 323 us);
-    // unequal ranges, wave priorities falling with progress and one workgroup
-    // per CU were each slower (per-workgroup timestamps: the second workgroup
-    // on a CU runs its equal range 15-20 % slower than the first).  Two
-    // partial slots per workgroup.
-    const size_t sk_bytes = (size_t)2 * slots * 16 * pl.mb * gemm::kThreads * 4;
-    if (pl.mb == 8 && tiles < slots && tiles * 2 >= slots && workspace_len >= 1 + tiles &&
-        sk_bytes < ((size_t)1 << 31) && (int64_t)groups * tiles < ((int64_t)1 << 31)) {
-      pl.sk_wgs = (int)slots;
-      pl.full_tiles = 0;
-      pl.tail_tiles = (int)tiles;
-      pl.tail_splits = 1;
-      pl.wgs = slots;
-      pl.partial_bytes = align_up(sk_bytes);
-      pl.keys_bytes = align_up((size_t)m * (size_t)pl.n_cg * 8);
-      return pl;
-    }
     pl.full_tiles = (int)full;
     pl.tail_tiles = (int)tail;
     pl.tail_splits = s;
     pl.wgs = full + tail * s;
     pl.partial_bytes = tail > 0 ? align_up((size_t)tail * s * 16 * pl.mb * gemm::kThreads * 4) : 0;
+    return pl;
   }
   pl.keys_bytes = align_up((size_t)m * (size_t)pl.n_cg * 8);
   return pl;
@@ -473,6 +541,7 @@ inline Plan make_plan(int64_t m, int64_t n, int64_t k, int64_t workspace_len, bo
 inline int64_t counters_needed(const Plan& pl, bool argmax) {
   // plain stores on wide tiles count per 64-column chunk (see skinny::wave_epilogue)
   if (pl.skinny && pl.splits > 1) return 1 + (int64_t)pl.n_cg * (argmax ? 1 : pl.cpw == skinny::kWaves ? pl.cpw : 1);
+  if (!pl.skinny && pl.two_pass) return 0;
   if (!pl.skinny && pl.tail_tiles > 0) return 1 + (int64_t)pl.tail_tiles;  // stream-K: every tile
   return argmax ? 1 : 0;
 }
@@ -595,6 +664,7 @@ int run(Variant var, const uint16_t* a, const int32_t* b, uint16_t* c, const uin
   p.argmax_state = argmax_state; p.argmax_out = argmax_out;
   p.m = (int)m; p.n = (int)n; p.k = (int)k; p.grouped = grouped;
   p.full_tiles = pl.full_tiles; p.tail_splits = pl.tail_splits; p.sk_wgs = pl.sk_wgs;
+  p.two_pass = pl.two_pass ? 1 : 0;
   p.partial_bytes = (uint32_t)pl.partial_bytes;
   p.kp_total = (int)(k / 32); p.n_cg = pl.n_cg; p.n_mb = pl.n_mb;
   dim3 grid((unsigned)pl.wgs, 1, 1);
@@ -622,6 +692,22 @@ int run(Variant var, const uint16_t* a, const int32_t* b, uint16_t* c, const uin
   } while (0)
   if (var == V_ARGMAX) LB_GM_MB(gemm::EPI_ARGMAX);
   else LB_GM_MB(gemm::EPI_STORE);
+  if (pl.two_pass) {
+    const dim3 blocks((unsigned)(pl.tail_tiles * 4 * pl.mb), 1, 1);
+#define LB_RED(MBV, GV)                                                                                            \
+  hipLaunchKernelGGL((gemm::reduce_kernel<MBV, GV>), blocks, dim3(gemm::kThreads), 0, st, partial, s, c, (int)m, \
+                     (int)n, pl.n_cg, pl.tail_splits)
+#define LB_RED_G(MBV)                  \
+  do {                                 \
+    if (grouped) LB_RED(MBV, true);    \
+    else LB_RED(MBV, false);           \
+  } while (0)
+    if (pl.mb == 8) LB_RED_G(8);
+    else if (pl.mb == 4) LB_RED_G(4);
+    else LB_RED_G(2);
+#undef LB_RED_G
+#undef LB_RED
+  }
 #undef LB_GM_MB
 #undef LB_GM_G
 #undef LB_GM
@@ -659,10 +745,11 @@ extern "C" size_t lb_marlin_scratch_bytes(int64_t prob_m, int64_t prob_n, int64_
   // (with and without the mixed plan, which only grouped scales take)
   const marlin::Plan a = marlin::make_plan(prob_m, prob_n, prob_k, INT64_MAX, false);
   const marlin::Plan a2 = marlin::make_plan(prob_m, prob_n, prob_k, INT64_MAX, false, false, false);
+  const marlin::Plan b2 = marlin::make_plan(prob_m, prob_n, prob_k, INT64_MAX, true, false, false);
   const marlin::Plan b = marlin::make_plan(prob_m, prob_n, prob_k, INT64_MAX, true);
   const marlin::Plan c = marlin::make_plan(prob_m, prob_n, prob_k, INT64_MAX, false, true);
   return std::max(std::max(std::max(a.partial_bytes + a.keys_bytes, a2.partial_bytes + a2.keys_bytes),
-                           b.partial_bytes + b.keys_bytes + b.act_bytes),
+                           std::max(b.partial_bytes, b2.partial_bytes) + b.keys_bytes + b.act_bytes),
                   c.partial_bytes + c.keys_bytes);
 }
 
@@ -830,7 +917,7 @@ FusedMlpPlan fused_mlp_plan(int64_t batch, int64_t hidden, int64_t inter, bool g
   // tiles that can pair gate and up chunks (its SiLU-gated store saves the
   // down launch's separate gating pass)
   p.up = marlin::make_plan(batch, 2 * inter, hidden, INT64_MAX, false, false,
-                           g1 && batch <= marlin::kMixedMaxM);
+                           g1, batch <= marlin::kMixedMaxM);
   p.down = marlin::make_plan(batch, hidden, inter, INT64_MAX, true, false, g2);
   // decode tiles of 2 or 4 chunks pair gate and up chunks; single-chunk tiles
   // and prefill tiles take the [g | u] round trip

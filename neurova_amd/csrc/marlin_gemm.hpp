@@ -61,6 +61,7 @@ struct Params {
   int grouped;
   int full_tiles;        // tiles computed whole, by workgroups 0 .. full_tiles - 1
   int tail_splits;       // the remaining tiles are split over K among this many workgroups each
+  int two_pass;          // split tiles only publish their partials; reduce_kernel sums them
   int sk_wgs;            // > 0: stream-K schedule over this many workgroups (full_tiles, tail_splits unused)
   int kp_total;
   int n_cg;
@@ -484,6 +485,7 @@ __global__ __launch_bounds__(kThreads, wgs_per_cu(MB)) void marlin_gemm_kernel(P
 #pragma unroll
       for (int i = 0; i < MB; ++i)
         publish16(rp, own_off + (uint32_t)(j * MB + i) * kRegBytes, acc[j][i]);
+    if (!SK && p.two_pass) return;
     wait_published();
     __syncthreads();
     int32_t* ctr = p.counters + ctr_idx;
@@ -652,6 +654,49 @@ __global__ __launch_bounds__(kThreads, wgs_per_cu(MB)) void marlin_gemm_kernel(P
   const int st0 = (int)(((int64_t)groups * split) / nsplit);           // first scale group (stage)
   const int nst = (int)(((int64_t)groups * (split + 1)) / nsplit) - st0;  // stages of this unit
   unit(tile, st0, nst, nsplit > 1, split);
+  }
+}
+
+// Sums the partials of a launch whose tiles are all split over K (two_pass)
+// in split order, rounds and stores.  Block (tile, accumulator register) of the
+// partial layout; thread: that register's four rows of one column.  The last
+// arrival of a tile would read all its splits alone, on one CU and with a
+// memory round trip for every few of them (M = 64, K = 17408, N = 5120, 10
+// splits: about 20 of 33 us); as a launch of its own the sum runs on every CU,
+// bound by the partials' bytes (S * M * N * 4, just written) and the launch.
+template <int MB, bool GROUPED>
+__global__ __launch_bounds__(kThreads) void reduce_kernel(const float* __restrict__ partial, const uint16_t* __restrict__ s,
+                                                          uint16_t* __restrict__ c, int m, int n, int n_cg, int splits) {
+  constexpr int kQ = 4 * MB;
+  constexpr int kBatch = 8;  // loads in flight
+  const int tile = blockIdx.x / kQ, q = blockIdx.x - tile * kQ;
+  const int mb = tile / n_cg, cg = tile - mb * n_cg;
+  const int j = q / MB, i = q - j * MB;
+  const int row0 = (mb * MB + i) * 16;
+  if (row0 >= m) return;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const f32x4* src = reinterpret_cast<const f32x4*>(partial) + ((int64_t)tile * splits * kQ + q) * kThreads + tid;
+  f32x4 sum = {0.f, 0.f, 0.f, 0.f};
+  for (int s0 = 0; s0 < splits; s0 += kBatch) {
+    f32x4 v[kBatch];
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u) v[u] = src[(int64_t)min(s0 + u, splits - 1) * kQ * kThreads];
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u)
+      if (s0 + u < splits) sum += v[u];
+  }
+  const int col = (cg * kWaves + (tid >> 6)) * 64 + 16 * j + (lane & 15);
+  const int row = row0 + 4 * (lane >> 4);
+  f16 cs = (f16)1.0f;
+  if (!GROUPED) {
+    const int r = col & 31;
+    cs = __builtin_bit_cast(f16, s[(col & ~31) + 8 * ((r >> 1) & 3) + ((r >> 3) << 1) + (r & 1)]);
+  }
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    f16 h = (f16)sum[e];
+    if (!GROUPED) h = h * cs;
+    if (row + e < m) c[(int64_t)(row + e) * n + col] = __builtin_bit_cast(uint16_t, h);
   }
 }
 

@@ -1,0 +1,99 @@
+"""Prefill plans below one round of 128-row tiles: the tile heights and k
+splits the planner chooses, with the split sums made by a second launch, and
+whole tiles where the stream-K schedule was; plain and SiLU-gated A, both
+scale modes, ragged last row blocks, every output against the oracle."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from oracle import lowbit_oracle as O
+from tests.gpu_util import assert_close_f16, assert_reference_rounding, print_case, to_dev, to_np
+
+pytestmark = pytest.mark.gpu
+
+
+def _buffers(dev, m, n, k, g):
+    import torch
+    from neurova_amd import capi
+
+    c = torch.full((m, n), float("nan"), dtype=torch.float16, device=dev)
+    ws = torch.zeros((n // 128 * 16,), dtype=torch.int32, device=dev)
+    # partials start as NaN: every one that is summed has to be written first
+    sc = torch.full((capi.marlin_scratch_bytes(m, n, k, g),), 255, dtype=torch.uint8, device=dev)
+    return c, ws, sc
+
+
+@pytest.mark.parametrize("m,k,n,group,height,split", [
+    (33, 2560, 1280, 128, 2, True),    # 32-row tiles, the last one of a single row
+    (65, 1024, 2048, -1, 2, True),
+    (40, 5120, 14336, 128, 4, True),   # 64-row tiles
+    (180, 2048, 5120, -1, 4, True),
+    (200, 5120, 7168, 128, 8, True),   # 128-row tiles split over K
+    (200, 5120, 5120, 128, None, True),
+    (1000, 2304, 9216, 128, 8, False),  # 288 whole tiles, 96 rows of the last block missing
+    (40, 256, 512, 128, None, None),    # two scale groups
+])
+def test_shapes_vs_oracle(dev, m, k, n, group, height, split):
+    import torch
+    from neurova_amd import capi
+
+    plan = capi.marlin_describe_plan(m, n, k, group)
+    assert plan["form"] == "prefill", plan
+    if height is not None:
+        assert plan["chunks_or_row_blocks"] == height, plan
+    if split is not None:
+        assert (plan["splits"] > 1) == split and (plan["row_blocks_or_full_tiles"] == 0) == split, plan
+    print_case("gemm-shape", m, k, n, group)
+    codes, qw, _, sp, x = O.make_marlin_inputs(m, k, n, group, seed=3000 + m + k)
+    c, ws, sc = _buffers(dev, m, n, k, group)
+    a, b, s = to_dev(x, dev), to_dev(qw, dev), to_dev(sp, dev)
+    got = []
+    for _ in range(2):
+        assert capi.marlin_gemm(a, b, c, s, ws, group, sc) == 0
+        torch.cuda.synchronize()
+        got.append(to_np(c).copy())
+    ref = O.marlin_gemm(x, qw, sp, group)
+    assert_close_f16(got[0], ref, what=f"m={m} k={k} n={n} g={group}")
+    if group == 128:
+        assert_reference_rounding(got[0], ref, x, qw, sp, group, what=f"m={m} k={k} n={n}")
+    assert np.array_equal(got[0].view(np.uint16), got[1].view(np.uint16))
+    assert int(ws.abs().sum()) == 0
+
+
+@pytest.mark.parametrize("m,k,n", [(33, 1024, 768), (70, 2048, 1280), (130, 3072, 512), (260, 1024, 1280), (1100, 1024, 8448)])
+def test_silu_packed_prefill_vs_oracle(dev, m, k, n):
+    """The gated activations are formed once in scratch; the product over them
+    takes the plain plans."""
+    import torch
+    from neurova_amd import capi
+
+    print_case("silu-prefill", m, k, n)
+    _, qw, _, sp, _ = O.make_marlin_inputs(m, k, n, 128, seed=3100 + m)
+    mixed = np.random.default_rng(3100 + m).normal(0, 1, (m, 2 * k)).astype(np.float16)
+    c, ws, sc = _buffers(dev, m, n, k, 128)
+    assert capi.marlin_gemm_silu_packed(to_dev(mixed, dev), to_dev(qw, dev), c, to_dev(sp, dev), ws, 128, sc) == 0
+    torch.cuda.synchronize()
+    assert int(ws.abs().sum()) == 0
+    assert_close_f16(to_np(c), O.marlin_gemm_silu_packed(mixed, qw, sp, k, 128), what=f"silu m={m}")
+
+
+@pytest.mark.parametrize("m", [48, 300])
+def test_workspace_of_one_entry(dev, m):
+    """Plans whose splits are summed by a second launch use no workspace
+    counters: the smallest workspace gives the same outputs."""
+    import torch
+    from neurova_amd import capi
+
+    k, n = 2048, 2048
+    print_case("one-entry workspace", m)
+    _, qw, _, sp, x = O.make_marlin_inputs(m, k, n, 128, seed=3200 + m)
+    a, b, s = to_dev(x, dev), to_dev(qw, dev), to_dev(sp, dev)
+    outs = []
+    for entries in (n // 128 * 16, 1):
+        c, _, sc = _buffers(dev, m, n, k, 128)
+        ws = torch.zeros((entries,), dtype=torch.int32, device=dev)
+        assert capi.marlin_gemm(a, b, c, s, ws, 128, sc) == 0
+        torch.cuda.synchronize()
+        outs.append(to_np(c))
+    assert np.array_equal(outs[0].view(np.uint16), outs[1].view(np.uint16))
