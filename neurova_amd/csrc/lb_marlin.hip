@@ -366,6 +366,11 @@ constexpr int64_t kMixedMaxM = 4;      // rows with the A slice staged (measured
 constexpr int64_t kMixedDirectMaxM = 32;    // rows with A loaded per step, one whole-K tile per CU
 constexpr int64_t kMixedDirectMaxM2 = 8;    // ... and with two whole-K tiles per CU
 
+// Where the direct form's A goes through the waves' own LDS (skinny::A_WAVE): at
+// M = 28 the two are even at K = 5120, N = 5120 (11.8 us) and with a short K a
+// wave runs too few batches for it (M = 28, K = 2048, N = 3072 9.1 against 8.9 us).
+inline bool wave_a(int64_t m, int64_t k) { return m > 28 && k >= 4096; }
+
 inline Plan make_plan(int64_t m, int64_t n, int64_t k, int64_t workspace_len, bool gated, bool argmax = false,
                       bool grouped = true, bool allow_mixed = true) {
   Plan pl;
@@ -420,7 +425,8 @@ inline Plan make_plan(int64_t m, int64_t n, int64_t k, int64_t workspace_len, bo
         pl.whole = (int)whole;
         pl.splits = s;
         pl.x_bytes = mixed_direct ? 0 : (size_t)groups * 128 * (size_t)m * 2;
-        pl.lds = std::max(mixed_direct ? 0 : pl.x_bytes + 16, (size_t)m * skinny::kCols * 4);
+        pl.lds = std::max(!mixed_direct ? pl.x_bytes + 16 : wave_a(m, k) ? (size_t)skinny::wave_a_bytes(pl.mr) : 0,
+                          (size_t)m * skinny::kCols * 4);
         pl.partial_bytes = left > 0 ? align_up((size_t)s * (size_t)m * (size_t)n * 4) : 0;
         pl.keys_bytes = align_up((size_t)m * (size_t)pl.n_cg * 8);
         return pl;
@@ -453,7 +459,8 @@ inline Plan make_plan(int64_t m, int64_t n, int64_t k, int64_t workspace_len, bo
     const size_t tile = (direct && cpw == skinny::kWaves) ? 0 : (size_t)m * skinny::kCols * 4;
     // A_RING: two batches of [M][128 k] in fragment order + the zero entry
     const size_t ring = (direct && cpw == skinny::kWaves) ? (size_t)(32 * m + 1) * 16 : 0;
-    pl.lds = std::max(std::max(stage, tile), ring);
+    const size_t wave = (direct && cpw != skinny::kWaves && wave_a(m, k)) ? (size_t)skinny::wave_a_bytes(pl.mr) : 0;
+    pl.lds = std::max(std::max(stage, tile), std::max(ring, wave));
     pl.partial_bytes = pl.splits > 1 ? align_up((size_t)pl.splits * (size_t)m * (size_t)n * 4) : 0;
     if (direct && gated) pl.act_bytes = align_up((size_t)m * (size_t)k * 2);
   } else {
@@ -620,8 +627,10 @@ int run(Variant var, const uint16_t* a, const int32_t* b, uint16_t* c, const uin
     } else if (pl.mr == 1) {
       if (pl.cpw == 2) LB_SKDG(skinny::A_DIRECT, 2, 1);
       else LB_SKDG(skinny::A_DIRECT, 1, 1);
-    } else {  // M = 17..32: 64-column tiles (make_plan)
+    } else if (!wave_a(m, k)) {  // M = 17..32: 64-column tiles (make_plan)
       LB_SKDG(skinny::A_DIRECT, 1, 2);
+    } else {
+      LB_SKDG(skinny::A_WAVE, 1, 2);
     }
 #undef LB_SKDG
 #undef LB_SKD

@@ -74,7 +74,11 @@ constexpr int kDepth = 2;               // weight batches in flight
 // A_DIRECT: plain fp16 A, not staged: fragments loaded per step (M up to 32).
 // A_RING: plain fp16 A staged one batch (one scale group) at a time through a
 // two-slot LDS ring, for 4-chunk tiles whose waves share it (M up to 32).
-enum AMode { A_PLAIN = 0, A_SILU_PACKED = 1, A_DIRECT = 3, A_RING = 4 };
+// A_WAVE: as A_DIRECT, each wave's batch of A through LDS of its own (M = 29..32).
+enum AMode { A_PLAIN = 0, A_SILU_PACKED = 1, A_DIRECT = 3, A_RING = 4, A_WAVE = 5 };
+constexpr int kWaveRowBytes = 17 * 16;  // A_WAVE: one LDS row of a batch, 128 k and 16 bytes of padding
+// dynamic LDS of an A_WAVE workgroup of `mr` 16-row blocks
+__host__ __device__ constexpr int wave_a_bytes(int mr) { return kWaves * 16 * mr * kWaveRowBytes; }
 // EPI_ACT: the tile pairs gate and up chunks (gate_up projection of an MLP)
 // and stores fp16(silu(g) * u) of its fp16 outputs instead of the outputs.
 enum EpiMode { EPI_STORE = 0, EPI_ARGMAX = 1, EPI_ACT = 2 };
@@ -309,12 +313,13 @@ __device__ __forceinline__ bool wave_epilogue(const Params& p, const f32x4 (&acc
 template <int AM, int EPI, bool GROUPED, int CPW, int MR = 1>
 __device__ __forceinline__ bool skinny_tile(const Params p, const int cg, const int split) {
   static_assert(EPI != EPI_ACT || CPW >= 2, "EPI_ACT pairs a gate and an up chunk");
-  static_assert(MR == 1 || ((AM == A_DIRECT || AM == A_RING) && (EPI == EPI_STORE || EPI == EPI_ACT)),
+  static_assert(MR == 1 || ((AM == A_DIRECT || AM == A_RING || AM == A_WAVE) && (EPI == EPI_STORE || EPI == EPI_ACT)),
                 "row blocks > 1: direct or ring A, store or SiLU-gated epilogue");
   static_assert(MR >= 1 && MR <= kMaxMR, "row blocks");
   static_assert(AM != A_RING || (CPW == kWaves && EPI != EPI_ARGMAX), "A ring: 4-chunk tiles");
   constexpr bool kDirect = AM == A_DIRECT;
   constexpr bool kRing = AM == A_RING;
+  constexpr bool kWaveA = AM == A_WAVE;
   constexpr int kRows = 16 * MR;  // rows of the MFMA tile
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   __shared__ int s_prev;
@@ -458,10 +463,40 @@ __device__ __forceinline__ bool skinny_tile(const Params p, const int cg, const 
     }
   };
 
+  // A_WAVE: with A_DIRECT's loads neighbouring lanes read different rows, and
+  // every row a sixteen-lane group touches is a cache-line access of its own
+  // (M = 16: 64 a load instruction).  Here load u of a lane is the 16 bytes at
+  // octet lane & 15 of row 4 u + (lane >> 4) of the batch (four rows of 256
+  // contiguous bytes an instruction, 8 cache lines), and the fragments come from
+  // the wave's own LDS rows: halves 4 gq .. + 3 and 8 + 4 gq .. + 3 of a k16 row
+  // are two 8-byte reads 16 bytes apart, which the padding spreads over all
+  // banks.  No barrier: a wave reads what it stored.  The LDS round trip pays
+  // near the full 32 rows (M = 32: K = 5120, N = 14336 19.5 -> 17.3 us, N = 7168
+  // 14.8 -> 13.9, K = 17408, N = 5120 23.8 -> 22.1; M = 24 even; M = 16 and below
+  // up to 10 % slower, also where only two workgroups per CU were asked for).
+  char* const wa = reinterpret_cast<char*>(smem) + wave * (kRows * kWaveRowBytes);
+  uint32_t aoff[4 * MR];
+  if constexpr (kWaveA) {
+#pragma unroll
+    for (int u = 0; u < 4 * MR; ++u)
+      aoff[u] = ((uint32_t)min(4 * u + g, mrows - 1) * (uint32_t)p.k + 8u * (uint32_t)mrow) * 2u;
+  }
+  auto wave_store = [&](const u32x4(&src)[kSteps][MR]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < 4 * MR; ++u)
+      *reinterpret_cast<u32x4*>(wa + (4 * u + g) * kWaveRowBytes + 16 * mrow) = src[u / MR][u % MR];
+    asm volatile("" ::: "memory");  // the reads that follow are of other lanes' stores
+  };
+  auto wave_frag = [&](int rb, int d) __attribute__((always_inline)) {
+    const char* src = wa + (16 * rb + mrow) * kWaveRowBytes + 64 * d + 32 * prow + 8 * gq;
+    const u32x2 lo = *reinterpret_cast<const u32x2*>(src), hi = *reinterpret_cast<const u32x2*>(src + 16);
+    return __builtin_bit_cast(f16x8, (u32x4){lo[0], lo[1], hi[0], hi[1]});
+  };
+
   // Ring of kDepth batches (one scale group, 1 KB per wave, each) in flight.
   u32x4 bw[kDepth][kSteps];
   u32x4 bs[kDepth];
-  u32x4 aw[kDepth][kSteps][MR];  // A_DIRECT only
+  u32x4 aw[kDepth][kSteps][MR];  // A_DIRECT: [step][row block]; A_WAVE: load u at [u / MR][u % MR]
 #pragma unroll
   for (int i = 0; i < kDepth; ++i) bs[i] = (u32x4){0, 0, 0, 0};
   auto issue_step = [&](int slot, int batch, int d) __attribute__((always_inline)) {
@@ -473,6 +508,11 @@ __device__ __forceinline__ bool skinny_tile(const Params p, const int cg, const 
       for (int rb = 0; rb < MR; ++rb) aw[slot][d][rb] = *reinterpret_cast<const u32x4*>(arow[rb] + 32 * (kpf + d));
     }
   };
+  auto issue_wave_a = [&](int slot, int batch) __attribute__((always_inline)) {
+    const char* base = reinterpret_cast<const char*>(p.a) + (size_t)((uint32_t)(kpw0 + batch * kSteps) * 64u);  // uniform
+#pragma unroll
+    for (int u = 0; u < 4 * MR; ++u) aw[slot][u / MR][u % MR] = *reinterpret_cast<const u32x4*>(base + aoff[u]);
+  };
   auto issue_scale = [&](int slot, int batch) __attribute__((always_inline)) {
     const int kpf = kpw0 + batch * kSteps;
     if (GROUPED)
@@ -481,13 +521,14 @@ __device__ __forceinline__ bool skinny_tile(const Params p, const int cg, const 
   auto issue = [&](int slot, int batch) __attribute__((always_inline)) {
 #pragma unroll
     for (int d = 0; d < kSteps; ++d) issue_step(slot, batch, d);
+    if constexpr (kWaveA) issue_wave_a(slot, batch);
     issue_scale(slot, batch);
   };
 
   // ---- staging loads, then the first weight batches, then the stores ----
   // (A_DIRECT: no staging; A_RING: batch 0 of A, then per weight batch i the
   // A batch i + 1)
-  if (!kDirect && !kRing) stage_load(0);
+  if (!kDirect && !kRing && !kWaveA) stage_load(0);
   if constexpr (kRing) ring_load(ar0, 0);
   __builtin_amdgcn_sched_barrier(0);  // staging loads strictly before the weight loads
 #pragma unroll
@@ -502,7 +543,7 @@ __device__ __forceinline__ bool skinny_tile(const Params p, const int cg, const 
     if (tid == 0) afr[ring_zero] = (u32x4){0, 0, 0, 0};
     lds_barrier();  // LDS only: the weight ring stays in flight
   }
-  if constexpr (!kDirect && !kRing) {
+  if constexpr (!kDirect && !kRing && !kWaveA) {
     __builtin_amdgcn_sched_barrier(0);
     stage_store(0);
     for (int base = kThreads * kStageUnroll; base < items; base += kThreads * kStageUnroll) {
@@ -548,10 +589,14 @@ __device__ __forceinline__ bool skinny_tile(const Params p, const int cg, const 
       const f16 s = __builtin_bit_cast(f16, (uint16_t)(scl[j] >> (16 * hsel)));
       sc2[j] = (f16x2){s, s};
     }
+    if constexpr (kWaveA) wave_store(aw[slot]);
 #pragma unroll
     for (int d = 0; d < kSteps; ++d) {
       f16x8 afrag[MR];
-      if constexpr (kDirect) {
+      if constexpr (kWaveA) {
+#pragma unroll
+        for (int rb = 0; rb < MR; ++rb) afrag[rb] = wave_frag(rb, d);
+      } else if constexpr (kDirect) {
 #pragma unroll
         for (int rb = 0; rb < MR; ++rb) {
           // odd rows of word 0 (gq = 1: halves 8, 9) <-> even rows of word 2
@@ -588,6 +633,7 @@ __device__ __forceinline__ bool skinny_tile(const Params p, const int cg, const 
           acc[rb][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(afrag[rb], bfrag, acc[rb][j], 0, 0, 0);
       }
     }
+    if constexpr (kWaveA) asm volatile("" ::: "memory");  // the next batch's stores stay behind these reads
   };
 
   // Full rounds re-issue every slot kDepth batches ahead; the tail (fewer than

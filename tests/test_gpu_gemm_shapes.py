@@ -78,6 +78,28 @@ def test_silu_packed_prefill_vs_oracle(dev, m, k, n):
     assert_close_f16(to_np(c), O.marlin_gemm_silu_packed(mixed, qw, sp, k, 128), what=f"silu m={m}")
 
 
+@pytest.mark.parametrize("m,k,n,group", [(29, 4096, 2048, 128), (31, 5120, 5120, -1), (32, 4224, 1280, 128),
+                                         (30, 5120, 14336, 128), (28, 4096, 2048, 128)])
+def test_wave_staged_decode_vs_oracle(dev, m, k, n, group):
+    """M = 29..32 with a long K: each wave's batches of A go through its own LDS
+    (M = 28: loaded as fragments); split and whole-K tiles, both scale modes."""
+    import torch
+    from neurova_amd import capi
+
+    plan = capi.marlin_describe_plan(m, n, k, group)
+    assert plan["form"] == "direct" and (plan["lds_bytes"] >= 4 * 32 * 272) == (m > 28), plan
+    print_case("wave-staged", m, k, n, group)
+    _, qw, _, sp, x = O.make_marlin_inputs(m, k, n, group, seed=3300 + m + k)
+    c, ws, sc = _buffers(dev, m, n, k, group)
+    assert capi.marlin_gemm(to_dev(x, dev), to_dev(qw, dev), c, to_dev(sp, dev), ws, group, sc) == 0
+    torch.cuda.synchronize()
+    ref = O.marlin_gemm(x, qw, sp, group)
+    assert_close_f16(to_np(c), ref, what=f"m={m} k={k} n={n} g={group}")
+    if group == 128:
+        assert_reference_rounding(to_np(c), ref, x, qw, sp, group, what=f"m={m} k={k} n={n}")
+    assert int(ws.abs().sum()) == 0
+
+
 @pytest.mark.parametrize("m", [48, 300])
 def test_workspace_of_one_entry(dev, m):
     """Plans whose splits are summed by a second launch use no workspace
