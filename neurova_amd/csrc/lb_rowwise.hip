@@ -5,8 +5,8 @@
 // qweight is an LSB-first bitstream, code c at bits [c*b, c*b+b); value
 // (code - 2^(b-1)) * scale[r, c / group] (csrc/lowbit_gemv.cu:4-14, 16-70).
 //
-// One activation row of whole 32-code units: rowwise_lds_kernel (2, 3, 4, 8
-// bits), rowwise_fast_kernel otherwise.  Batches and ragged rows: the matrix-core
+// One activation row of whole 32-code units: rowwise_lds_kernel, or
+// rowwise_fast_kernel for rows and groups it does not take.  Batches and ragged rows: the matrix-core
 // product (rowwise_mm.hpp).  rowwise_general_kernel takes the rest (groups that
 // are no multiple of 32 columns), reading bytes like the reference's scalar
 // decode.
@@ -134,11 +134,11 @@ __global__ __launch_bounds__(kThreads) void rowwise_fast_kernel(Params p) {
 }
 
 // ---------------------------------------------------------------------------
-// Single-row GEMV with the activation row staged in LDS (batch 1, 2/3/4/8 bits,
-// columns a multiple of 32).
+// Single-row GEMV with the activation row staged in LDS (batch 1, columns a
+// multiple of 32).
 //
-// A 32-code unit (BITS dwords) is decoded into 16 fp16 pairs with one AND per
-// pair: two codes that sit at the same bit offset `off` of the two 16-bit
+// A 32-code unit (BITS dwords) is decoded into 16 fp16 pairs, at 2, 3, 4 and 8
+// bits with one AND per pair: two codes that sit at the same bit offset `off` of the two 16-bit
 // halves of a word (after at most one shift, bit-field insert, align or byte
 // permute) are kept as they lie, which read as the fp16 subnormals
 // (c * 2^off * 2^-24, c' * 2^off * 2^-24), exact.  The workgroup stages the
@@ -172,11 +172,11 @@ constexpr int kLdsPreMax8 = 1;
 __host__ __device__ constexpr int pair_lo(int bits, int q) {
   return bits == 2 ? 16 * (q >> 3) + (q & 7)
        : bits == 3 ? (q < 5 ? q : q < 9 ? q + 1 : q < 14 ? q + 2 : (q == 14 ? 5 : 10))
-       : bits == 4 ? 8 * (q >> 2) + (q & 3)
+       : bits <= 7 ? 8 * (q >> 2) + (q & 3)
        : 4 * (q >> 1) + (q & 1);
 }
 __host__ __device__ constexpr int pair_hi(int bits, int q) {
-  return bits == 2 ? pair_lo(2, q) + 8 : bits == 3 ? pair_lo(3, q) + 16 : bits == 4 ? pair_lo(4, q) + 4 : pair_lo(8, q) + 2;
+  return bits == 2 ? pair_lo(2, q) + 8 : bits == 3 ? pair_lo(3, q) + 16 : bits <= 7 ? pair_lo(4, q) + 4 : pair_lo(8, q) + 2;
 }
 // Offset classes: b2 {0,2,4,6,8}, b3 {1,4,7}, b4 {0,4}, b8 {0}.  v_dot2_f32_f16
 // keeps fewer bits of a product the more leading zeros a subnormal factor has,
@@ -191,16 +191,62 @@ __host__ __device__ constexpr int off_of_class(int bits, int c) {
   return bits == 2 ? 2 * c : bits == 3 ? 3 * c + 1 : bits == 4 ? 4 * c : c;
 }
 __host__ __device__ constexpr int pair_off(int bits, int q) {
-  return bits == 2 ? ((q & 7) < 5 ? 2 * (q & 7) : 2 * (q & 7) - 6)
+  return bits >= 5 ? 0
+       : bits == 2 ? ((q & 7) < 5 ? 2 * (q & 7) : 2 * (q & 7) - 6)
        : bits == 3 ? (q == 2 || q == 4 || q == 11 || q == 13 ? 7
                       : q == 1 || q == 3 || q == 6 || q == 8 || q == 10 || q == 12 ? 4 : 1)
        : bits == 4 ? 4 * (q & 1)
        : 0;
 }
 
+// 5, 6 and 7 bits: two codes a half leave no common offset, so their pairs
+// are decoded to the fp16 (code - z) itself: one class, no zero-point share.
+__host__ __device__ constexpr bool centered(int bits) { return bits >= 5 && bits <= 7; }
+
+// The 32 bits of the unit from bit P on (zeros past its end)).
+template <int BITS, int P>
+__device__ __forceinline__ uint32_t unit_window(const uint32_t* w) {
+  constexpr int d = P >> 5, s = P & 31;
+  if constexpr (s == 0) return w[d];
+  else if constexpr (d + 1 < BITS) return __builtin_amdgcn_alignbit(w[d + 1], w[d], s);
+  else return w[d] >> s;
+}
+
+// Codes 8 B .. 8 B + 7 of a unit of 5, 6 or 7 bits as the pairs (i, i + 4): two
+// words whose halves hold two codes each (three VALU), the second code of a half
+// shifted down where the two do not fit the ten mantissa bits, and per pair one
+// v_and_or under the exponent of 1024 and one packed add or fma.
+template <int BITS, int B>
+__device__ __forceinline__ void decode_block(const uint32_t* w, uint32_t* b, uint32_t magic) {
+  constexpr int P = 8 * BITS * B;
+  constexpr uint32_t m = (1u << BITS) - 1u, lo = m | (m << 16);
+  constexpr float zb = 1024.f + (float)(1 << (BITS - 1));
+  const uint32_t v01 = (unit_window<BITS, P>(w) & 0xffffu) | (unit_window<BITS, P + 4 * BITS - 16>(w) & 0xffff0000u);
+  const uint32_t v23 =
+      (unit_window<BITS, P + 2 * BITS>(w) & 0xffffu) | (unit_window<BITS, P + 6 * BITS - 16>(w) & 0xffff0000u);
+  const f16x2 bias = {(f16)zb, (f16)zb};
+  b[0] = as_u32(as_h2(and_or(v01, lo, magic)) - bias);
+  b[2] = as_u32(as_h2(and_or(v23, lo, magic)) - bias);
+  if constexpr (BITS == 5) {  // at offset 5: (1024 + 32 code) / 32 - (32 + z)
+    const f16x2 r = {(f16)0.03125f, (f16)0.03125f}, o = {(f16)-48.0f, (f16)-48.0f};
+    b[1] = as_u32(as_h2(and_or(v01, lo << 5, magic)) * r + o);
+    b[3] = as_u32(as_h2(and_or(v23, lo << 5, magic)) * r + o);
+  } else {
+    b[1] = as_u32(as_h2(and_or(v01 >> BITS, lo, magic)) - bias);
+    b[3] = as_u32(as_h2(and_or(v23 >> BITS, lo, magic)) - bias);
+  }
+}
+
 template <int BITS>
 __device__ __forceinline__ void decode_unit(const uint32_t* w, uint32_t (&b)[16]) {
-  if constexpr (BITS == 2) {
+  if constexpr (centered(BITS)) {
+    uint32_t magic;
+    asm("v_mov_b32 %0, 0x64006400" : "=v"(magic));
+    decode_block<BITS, 0>(w, b, magic);
+    decode_block<BITS, 1>(w, b + 4, magic);
+    decode_block<BITS, 2>(w, b + 8, magic);
+    decode_block<BITS, 3>(w, b + 12, magic);
+  } else if constexpr (BITS == 2) {
 #pragma unroll
     for (int d = 0; d < 2; ++d) {
       const uint32_t x = w[d], xs = x >> 6;
@@ -250,7 +296,7 @@ __device__ __forceinline__ void decode_unit(const uint32_t* w, uint32_t (&b)[16]
       b[4 * d + 3] = xs & 0x00f000f0u;
     }
   } else {
-    static_assert(BITS == 8, "2, 3, 4 or 8 bits");
+    static_assert(BITS == 8, "2 to 8 bits");
 #pragma unroll
     for (int d = 0; d < 8; ++d) {
       b[2 * d + 0] = w[d] & 0x00ff00ffu;
@@ -473,9 +519,11 @@ __global__ __launch_bounds__(W * kWave) void rowwise_lds_kernel(const uint8_t* q
             const int c = class_of_off(BITS, pair_off(BITS, q));
             tc[c] = __builtin_amdgcn_fdot2(as_h2(b[q]), as_h2(xq[q]), tc[c], false);
           }
-          float t = -cu;
+          float t = centered(BITS) ? tc[0] : -cu;
+          if constexpr (!centered(BITS)) {
 #pragma unroll
-          for (int c = 0; c < NC; ++c) t = __builtin_fmaf(tc[c], (float)(1 << (24 - off_of_class(BITS, c))), t);
+            for (int c = 0; c < NC; ++c) t = __builtin_fmaf(tc[c], (float)(1 << (24 - off_of_class(BITS, c))), t);
+          }
           acc[a][r] = __builtin_fmaf(t, sc[j][a][r], acc[a][r]);  // explicit: one rounding in every instantiation
         }
     }
@@ -644,7 +692,7 @@ int launch_lds_bits(const Params& p, hipStream_t st) {
   // resident at once.
   const int upl = (B == 2 && pairs) ? 2 : 1;
   const int64_t steps = ((p.cols >> 5) + upl * kWave - 1) / (upl * kWave);
-  const int cap = B == 8 ? kLdsPreMax8 : (NW == 1 ? kLdsPreMax : 5);
+  const int cap = B == 8 ? kLdsPreMax8 : centered(B) ? (steps <= 5 && R == 1 ? 5 : 1) : (NW == 1 ? kLdsPreMax : 5);
   const int64_t want = std::min<int64_t>(steps, cap);
   const int kp = want <= 1 ? 1 : want <= 2 ? 2 : want <= 3 ? 3 : want <= 5 ? 5 : 9;
   // two units per lane step: a last step of at most 32 units, when the
@@ -667,6 +715,15 @@ int launch_lds_bits(const Params& p, hipStream_t st) {
   } while (0)
   if constexpr (B == 8) {
     LB_LAUNCH(1, kLdsPreMax8);
+  } else if constexpr (centered(B)) {
+    if constexpr (R == 2) {
+      LB_LAUNCH(1, 1);
+    } else {
+      if (kp == 1) LB_LAUNCH(1, 1);
+      else if (kp == 2) LB_LAUNCH(1, 2);
+      else if (kp == 3) LB_LAUNCH(1, 3);
+      else LB_LAUNCH(1, 5);
+    }
   } else if constexpr (B == 2) {
     if (pairs && ht) {
       if (kp == 2) LB_LAUNCH_T(2, 2, true);
@@ -693,6 +750,11 @@ int launch_lds_bits(const Params& p, hipStream_t st) {
 // measured faster (one process, graph replay, against 8 waves of one row):
 //   8 bits, 5120 x 17408:  10 waves of 2 rows (256 workgroups) 18.5 us against 21.2 us;
 //   4 bits, 4096 x 4096:   16 waves of 1 row  (256 workgroups)  3.66 us against 3.95 us.
+// 5, 6 and 7 bits, against the fast kernel: 8 waves of one row with the whole row
+// prefetched up to five lane steps (5120 columns x 17408 rows: 22.5 -> 16.8, 23.6 ->
+// 18.4, 25.2 -> 20.1 us; 16 waves 18.3 to 22.1, one step prefetched 18.0 to 20.6),
+// beyond that 10 waves of two rows with one step (17408 x 5120: 21.8 -> 17.4, 23.4 ->
+// 18.3, 25.9 -> 19.8 us; 8 waves of one row 18.4 to 22.4).
 // 2 and 3 bits keep 8 waves of one row (2.5 workgroups per CU): every other
 // shape measured slower there (10 waves of 1 or 2 rows by 11-15 %, 16 waves by
 // 25-30 %, 8 waves of 2 rows by 27-38 %).
@@ -702,12 +764,19 @@ int launch_lds(const Params& p, int bits, hipStream_t st) {
     const int64_t cus = lbh::device_cus();
     if (bits == 8 && p.rows >= 20 * cus) return launch_lds_bits<8, 1, 10, 2>(p, st);
     if (bits == 4 && p.rows >= 16 * cus) return launch_lds_bits<4, 1, 16, 1>(p, st);
+    const bool tall = p.cols > 5 * 32 * kWave && p.rows >= 20 * cus;  // 5 to 7 bits, more than five lane steps
+    if (bits == 5 && tall) return launch_lds_bits<5, 1, 10, 2>(p, st);
+    if (bits == 6 && tall) return launch_lds_bits<6, 1, 10, 2>(p, st);
+    if (bits == 7 && tall) return launch_lds_bits<7, 1, 10, 2>(p, st);
   }
   constexpr int R = NW == 1 ? kLdsRows : (kLdsRows + 1) / 2;
   switch (bits) {
     case 2: return launch_lds_bits<2, NW, kLdsWaves, R>(p, st);
     case 3: return launch_lds_bits<3, NW, kLdsWaves, R>(p, st);
     case 4: return launch_lds_bits<4, NW, kLdsWaves, R>(p, st);
+    case 5: return launch_lds_bits<5, NW, kLdsWaves, R>(p, st);
+    case 6: return launch_lds_bits<6, NW, kLdsWaves, R>(p, st);
+    case 7: return launch_lds_bits<7, NW, kLdsWaves, R>(p, st);
     case 8: return launch_lds_bits<8, NW, kLdsWaves, R>(p, st);
     default: return LB_ERR_ARG;
   }
@@ -760,18 +829,18 @@ int launch_mm(const Params& p, int nw, int bits, hipStream_t st) {
 }
 
 // Whole 32-code units of one activation row: the LDS-staged kernel, or the fast
-// kernel at the widths and sizes that one does not take (5, 6, 7 bits at K =
-// 5120, N = 17408: 22.3 / 23.6 / 25.8 us, the matrix-core product 23.1 / 23.0 /
-// 27.7).  Everything else goes to the matrix-core product (ragged rows at that
+// kernel where the row does not fit LDS or the group is not a power of two of
+// units (g96 at 4 bits, K = 5120, N = 17408: 19.9 us, the matrix-core product
+// 20.9).  Everything else goes to the matrix-core product (ragged rows at that
 // size, 4 bits: 32.6 us against the general kernel's 132; a batch of 16 rows 26
-// against 196 us on four-row tiles of the fast kernel), except groups that
-// are neither a multiple of 32 columns nor the whole row: the general kernel.
+// against 196 us on four-row tiles of the fast kernel), except groups that are
+// neither a multiple of 32 columns nor the whole row: the general kernel.
 int launch(Params p, int nw, int bits, hipStream_t st) {
   const bool units = p.batch == 1 && p.cols % 32 == 0 && (p.packed_cols % 4 == 0) && lbh::aligned(p.q[0], 4) &&
                      (nw == 1 || lbh::aligned(p.q[1], 4)) && (p.group % 32 == 0) && lbh::aligned(p.x, 16);
   // staged in LDS
   const int64_t gu = p.group / 32;  // units per group
-  const bool lds = units && (bits == 2 || bits == 3 || bits == 4 || bits == 8) &&
+  const bool lds = units &&
                    (p.cols >> 5) * kLdsUnitBytes <= kLdsMaxBytes && (gu & (gu - 1)) == 0 &&
                    p.packed_cols * (p.rows > 0 ? 1 : 0) <= (int64_t)0xffffffff / 2 &&
                    p.rows < (int64_t(1) << 31) && p.scale_cols < (int64_t(1) << 31);  // int kernel arguments

@@ -87,3 +87,30 @@ def test_special_values(dev, bits):
     assert not np.isfinite(got[3]).any() and np.isnan(got[18]).all()
     keep = [i for i in range(20) if i not in (3, 18)]
     _check(got[keep], x[keep], packed, scales, cols, group, bits, f"b{bits}")
+
+
+@pytest.mark.parametrize("bits", [5, 6, 7])
+@pytest.mark.parametrize("rows,cols,group", [
+    (7, 32, 32), (9, 2016, 32), (16, 2080, 128), (5, 4128, 64), (33, 6176, 128), (8, 10240, 64), (3, 10272, 128),
+    (5127, 10272, 128), (5120, 10240, 64),  # two rows a wave above five lane steps, one below
+])
+def test_staged_row_of_whole_units(dev, bits, rows, cols, group):
+    """One activation row at 5, 6 and 7 bits, staged in LDS: one to five lane
+    steps prefetched, more than five, ragged last workgroups; the pair of
+    matrices equals two single calls."""
+    import torch
+    from neurova_amd import capi
+
+    print_case("staged-row", bits, rows, cols, group)
+    _, packed, scales, x = O.make_rowwise_inputs(rows, cols, bits, group, seed=bits + rows)
+    q, s, xd = to_dev(packed, dev), to_dev(scales, dev), to_dev(x[0], dev)
+    y = torch.full((rows,), float("nan"), dtype=torch.float16, device=dev)
+    assert capi.lowbit_gemv(q, s, xd, y, cols, group, bits) == 0
+    got = to_np(y)
+    _check(got.reshape(1, -1), x, packed, scales, cols, group, bits, f"b{bits}")
+    if rows < 100:
+        import langburst_cuda as lc
+
+        q2 = torch.flip(q, (0,)).contiguous()
+        a, b = lc.lowbit_gemv_pair(q, s, q2, s, xd, cols, group, bits)
+        assert torch.equal(a, y) and torch.equal(b, lc.lowbit_gemv(q2, s, xd, cols, group, bits))
