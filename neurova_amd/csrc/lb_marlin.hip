@@ -584,11 +584,22 @@ int run(Variant var, const uint16_t* a, const int32_t* b, uint16_t* c, const uin
   if (m > skinny::kMaxM && (a_bytes >= (1LL << 31) || k * n / 2 >= (1LL << 31))) return LB_ERR_PROB_SHAPE;
   if (k * n / 2 >= (1LL << 32)) return LB_ERR_PROB_SHAPE;
   const bool gated = var == V_SILU || var == V_SILU_DONE;
-  const Plan pl = make_plan(m, n, k, workspace_len, gated, var == V_ARGMAX,
-                            grouped != 0);
+  Plan pl = make_plan(m, n, k, workspace_len, gated, var == V_ARGMAX, grouped != 0);
+  // Without scratch for its partials a two-pass plan runs its tiles whole: a
+  // caller with a workspace too short for split counters could always call
+  // without scratch.
+  const size_t act_need = var == V_SILU ? pl.act_bytes : 0;
+  if (pl.two_pass && (!scratch || scratch_bytes < pl.partial_bytes + act_need)) {
+    pl.two_pass = false;
+    pl.full_tiles = pl.tail_tiles;
+    pl.tail_tiles = 0;
+    pl.tail_splits = 1;
+    pl.wgs = pl.full_tiles;
+    pl.partial_bytes = 0;
+  }
   if (var == V_SILU_DONE && !pl.skinny) return LB_ERR_ARG;  // decode batches only
   if (workspace_len < counters_needed(pl, var == V_ARGMAX)) return LB_ERR_WORKSPACE;
-  const size_t need = pl.partial_bytes + (var == V_ARGMAX ? pl.keys_bytes : 0) + (var == V_SILU ? pl.act_bytes : 0);
+  const size_t need = pl.partial_bytes + (var == V_ARGMAX ? pl.keys_bytes : 0) + act_need;
   if (need > 0 && (!scratch || scratch_bytes < need)) return LB_ERR_SCRATCH;
   if (need > 0 && !lbh::aligned(scratch, 16)) return LB_ERR_ALIGN;
 

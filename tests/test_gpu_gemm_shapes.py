@@ -119,3 +119,18 @@ def test_workspace_of_one_entry(dev, m):
         torch.cuda.synchronize()
         outs.append(to_np(c))
     assert np.array_equal(outs[0].view(np.uint16), outs[1].view(np.uint16))
+
+
+@pytest.mark.parametrize("m,k,n", [(20, 256, 512), (48, 2048, 2048), (300, 1024, 2048)])
+def test_one_entry_workspace_without_scratch(dev, m, k, n):
+    """With neither split counters nor scratch the tiles run whole."""
+    import torch
+    from neurova_amd import capi
+
+    print_case("no scratch", m, k, n)
+    _, qw, _, sp, x = O.make_marlin_inputs(m, k, n, 128, seed=3300 + m)
+    c, _, _ = _buffers(dev, m, n, k, 128)
+    ws = torch.zeros((1,), dtype=torch.int32, device=dev)
+    st = capi.marlin_gemm(to_dev(x, dev), to_dev(qw, dev), c, to_dev(sp, dev), ws, 128, None)
+    assert st == 0, capi.status_string(st)
+    assert_close_f16(to_np(c), O.marlin_gemm(x, qw, sp, 128), what=f"m={m} k={k} n={n}")
