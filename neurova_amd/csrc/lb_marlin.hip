@@ -490,7 +490,7 @@ inline Plan make_plan(int64_t m, int64_t n, int64_t k, int64_t workspace_len, bo
       const size_t sk_bytes = (size_t)2 * slots * 16 * 8 * gemm::kThreads * 4;
       const bool sk = tiles8 * 100 <= slots * 52 || (!grouped && k <= 2048) ||
                       (k > 8192 && tiles8 % 64 == 0 && tiles8 * 4 <= slots * 3);
-      if (sk && tiles8 * 2 >= slots && workspace_len >= 1 + tiles8 && sk_bytes < ((size_t)1 << 31) &&
+      if (sk && m >= 128 && tiles8 * 2 >= slots && workspace_len >= 1 + tiles8 && sk_bytes < ((size_t)1 << 31) &&
           (int64_t)groups * tiles8 < ((int64_t)1 << 31)) {
         pl.mb = 8;
         pl.n_mb = (int)((m + 127) / 128);

@@ -178,3 +178,10 @@ def test_noalloc_scratch_covers_decode_shapes(L, name):
     for m in range(1, 65):
         for g in (128, -1):
             assert capi.marlin_scratch_bytes(m, n, k, g) <= limit, (name, m, g)
+
+
+def test_prefill_below_128_rows_is_not_streamk(L):
+    """Stream-K runs 128-row tiles: wide projections of fewer rows keep lower ones."""
+    for m, n, k, g, variant in itertools.product((33, 40, 64, 100, 127), (65536, 66560, 81920), (1024, 5120, 17408), (128, -1), (0, 1)):
+        p = _plan(m, n, k, g, variant)
+        assert p["form"] == "prefill" and (m > 64 or p["chunks_or_row_blocks"] < 8), f"m={m} n={n} k={k} g={g}: {p}"
