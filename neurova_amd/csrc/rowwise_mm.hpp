@@ -235,12 +235,15 @@ struct Scales {
   __device__ __forceinline__ void init(const Params& p, int n0, int lane) {
     off = (uint32_t)min(n0 + min(lane, 16 * NB - 1), p.rows - 1) * (uint32_t)p.scale_cols * 2u;
   }
-  // (`last`: the last span that holds columns)
+  // (`last`: the last span that holds columns; spans past it count as scale 0,
+  // so that an infinity in the last group's scale stays one)
   __device__ __forceinline__ void load(uint16_t (&r)[SPS], const Params& p, const uint16_t* s, int stage, int last) const {
 #pragma unroll
-    for (int t = 0; t < SPS; ++t)
-      r[t] = *reinterpret_cast<const uint16_t*>(
+    for (int t = 0; t < SPS; ++t) {
+      const uint16_t v = *reinterpret_cast<const uint16_t*>(
           reinterpret_cast<const char*>(s + span_group(p, min(stage * SPS + t, last))) + off);
+      r[t] = stage * SPS + t <= last ? v : (uint16_t)0;
+    }
   }
   static __device__ __forceinline__ float get(uint16_t r, int j, int nl) {
     return h2f((uint16_t)__builtin_amdgcn_ds_bpermute((16 * j + nl) << 2, (int)(uint32_t)r));

@@ -89,6 +89,22 @@ def test_special_values(dev, bits):
     _check(got[keep], x[keep], packed, scales, cols, group, bits, f"b{bits}")
 
 
+@pytest.mark.parametrize("batch", [3, 40])
+@pytest.mark.parametrize("rows", [40, 16400])
+@pytest.mark.parametrize("cols,group", [(160, 32), (190, 64)])
+def test_infinite_scale_of_the_last_group(dev, batch, rows, cols, group):
+    """An infinite scale of a ragged row's last group gives infinities, not NaN."""
+    print_case("mm-inf-scale", batch, rows, cols, group)
+    _, packed, scales, x = O.make_rowwise_inputs(rows, cols, 4, group, batch=batch, seed=rows + batch)
+    scales[5, -1] = np.inf
+    got = _gemm(dev, packed, scales, np.abs(x) + np.float16(1), cols, group, 4)
+    w = O.rowwise_dequant_f32(packed, np.ones_like(scales), cols, group, 4).astype(np.float64)
+    last = cols - (scales.shape[1] - 1) * group
+    dot = (np.abs(x) + np.float16(1)).astype(np.float64)[:, -last:] @ w[5, -last:]
+    assert np.array_equal(got[:, 5], np.where(dot > 0, np.inf, -np.inf).astype(np.float16))
+    assert np.isfinite(np.delete(got, 5, axis=1)).all()
+
+
 @pytest.mark.parametrize("bits", [5, 6, 7])
 @pytest.mark.parametrize("rows,cols,group", [
     (7, 32, 32), (9, 2016, 32), (16, 2080, 128), (5, 4128, 64), (33, 6176, 128), (8, 10240, 64), (3, 10272, 128),
