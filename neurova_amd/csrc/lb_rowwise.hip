@@ -832,7 +832,7 @@ int launch_mm(const Params& p, int nw, int bits, hipStream_t st) {
 // kernel where the row does not fit LDS or the group is not a power of two of
 // units (g96 at 4 bits, K = 5120, N = 17408: 19.9 us, the matrix-core product
 // 20.9).  Everything else goes to the matrix-core product (ragged rows at that
-// size, 4 bits: 32.6 us against the general kernel's 132; a batch of 16 rows 26
+// size, 4 bits: 32.6 us against the general kernel's 132; a batch of 16 rows 21
 // against 196 us on four-row tiles of the fast kernel), except groups that are
 // neither a multiple of 32 columns nor the whole row: the general kernel.
 int launch(Params p, int nw, int bits, hipStream_t st) {

@@ -26,9 +26,21 @@ int launch_tile(const Params& p, hipStream_t st) {
 
 // Which form, from sweeps at 2, 3, 4 and 8 bits over M = 2..384, K x N = 5120 x
 // 17408 and 17408 x 5120 (times below: 4 bits, g128):
-//   up to 16 rows: 32 output rows per workgroup (M = 16: 25 us at N = 5120,
-//     16 rows 35 us, 64 rows 39 us), 16 where that leaves half the CUs idle;
-//   17 to 32: two blocks of 16 (M = 32, N = 5120: 31 us, one block 46);
+//   up to 16 rows: 32 output rows per workgroup (M = 16, N = 5120: 24 us, 16
+//     rows 34 us, 64 rows 38 us), 16 where that leaves half the CUs idle.  One
+//     stage in flight per wave: with two the registers leave room for one
+//     workgroup per CU instead of two (M = 16, N = 17408: 25.8 us against 22.5,
+//     8 bits 32.3 against 29.8).  Two in flight where there is one workgroup per
+//     CU at most anyway, few rows and few bits (K = 17408, N = 5120, M = 6: 19.8
+//     against 20.2 us; 2 bits 16.8 against 18.7 at M = 4, even at 16).
+//     More than two workgroups of 32 rows per CU: 48 rows from M = 9 on, up to
+//     4 bits (M = 16: N = 17408 22.5 -> 21.0 us, N = 34816 36.0 -> 31.4; M = 3
+//     16.3 against 17.2; 5 bits 26.0 against 26.5);
+//   17 to 32: two blocks of 16, eight waves and 32 rows (M = 32, N = 5120: 31
+//     us; 16 rows 46, four waves 45).  It is one workgroup per CU by its LDS, so
+//     with more than one for each four waves run (N = 14336 21.5 -> 20.5 us, K =
+//     2048, N = 16384 at 2 bits 12.2 -> 9.7), and with more than two 48 rows (N =
+//     17408 30.0 -> 25.7, N = 34816 48.4 -> 44.6; at N = 14336 25.1 against 20.5);
 //   above, where 64-column tiles of 64 rows do not give every CU one (N = 5120
 //     up to M = 192): four blocks of 16, the waves splitting K (M = 128: 72 us
 //     against 88 us); eight waves where that is one round of workgroups (M =
@@ -43,7 +55,13 @@ int launch_sps(const Params& p, int mats, hipStream_t st) {
     return (int64_t)((p.batch + 16 * mb - 1) / (16 * mb)) * ((p.rows + rows - 1) / rows) * mats;
   };
   if (p.batch <= 16) {
-    if (2 * wgs(1, 32) >= cus) return launch_skinny<SPS, 1, 2, 8, 2>(p, mats, st);
+    if constexpr (LB_RW_BITS <= 4) {
+      if (wgs(1, 32) > 2 * cus && p.batch > 8) return launch_skinny<SPS, 1, 3, 8, 1>(p, mats, st);
+      if constexpr (LB_RW_BITS == 2 || SPS == 1)
+        if (2 * wgs(1, 32) >= cus && wgs(1, 32) <= cus && (LB_RW_BITS == 2 || p.batch <= 8))
+          return launch_skinny<SPS, 1, 2, 8, 2>(p, mats, st);
+    }
+    if (2 * wgs(1, 32) >= cus) return launch_skinny<SPS, 1, 2, 8, 1>(p, mats, st);
     return launch_skinny<SPS, 1, 1, 8, 2>(p, mats, st);
   }
   const bool narrow = wgs(4, 64) < cus;
@@ -52,6 +70,8 @@ int launch_sps(const Params& p, int mats, hipStream_t st) {
       if (LB_RW_BITS <= 5 && wgs(4, 32) <= cus) return launch_skinny<SPS, 4, 2, LB_RW_BITS <= 5 ? 8 : 4, 1>(p, mats, st);
       return launch_skinny<SPS, 4, 2, 4, 1>(p, mats, st);
     }
+    if (wgs(2, 32) > 2 * cus) return launch_skinny<SPS, 2, 3, 4, 1>(p, mats, st);
+    if (wgs(2, 32) > cus) return launch_skinny<SPS, 2, 2, 4, 1>(p, mats, st);
     if (2 * wgs(2, 32) >= cus) return launch_skinny<SPS, 2, 2, 8, 1>(p, mats, st);
     if (2 * wgs(2, 16) >= cus) return launch_skinny<SPS, 2, 1, 8, 1>(p, mats, st);
     return launch_skinny<SPS, 1, 1, 8, 2>(p, mats, st);

@@ -28,7 +28,7 @@
 //
 // Measured (4 bits, g128, against the scalar-dot kernel that read and decoded
 // the weights again for every four batch rows): M = 16, K = 5120, N = 17408
-// 196 -> 26 us, K = 17408, N = 5120 186 -> 25 us; M = 384 at 2 bits, g64 4260 ->
+// 196 -> 21 us, K = 17408, N = 5120 186 -> 24 us; M = 384 at 2 bits, g64 4260 ->
 // 113 us and 3960 -> 125 us (604 TFLOP/s).  Up to 32 rows the few stages a wave
 // runs, their loads and the LDS traffic bound it (floor: 9.6 us of weight
 // bytes), above that the VALU work of the decode and the scales beside the MFMAs.

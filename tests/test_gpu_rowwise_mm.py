@@ -61,6 +61,18 @@ def test_launch_forms_vs_oracle(dev, batch, rows, bits, cols, group):
     _check(_gemm(dev, packed, scales, x, cols, group, bits), x, packed, scales, cols, group, bits, f"{batch}x{rows}")
 
 
+@pytest.mark.parametrize("batch", [8, 9, 17, 32])
+@pytest.mark.parametrize("rows", [8192, 8193, 16385])
+@pytest.mark.parametrize("bits,cols,group", [(2, 1152, 128), (4, 1300, 128), (3, 300, 32), (8, 257, 64)])
+def test_workgroups_per_cu_vs_oracle(dev, batch, rows, bits, cols, group):
+    """Up to one, up to two and more workgroups of 32 rows for each of 256 compute
+    units: blocks of 32 or 48 rows, four or eight waves, one or two stages in
+    flight, the last block of a single row."""
+    print_case("mm-cu", batch, rows, bits, cols, group)
+    _, packed, scales, x = O.make_rowwise_inputs(rows, cols, bits, group, batch=batch, seed=bits + rows + batch)
+    _check(_gemm(dev, packed, scales, x, cols, group, bits), x, packed, scales, cols, group, bits, f"{batch}x{rows}")
+
+
 @pytest.mark.parametrize("bits", [3, 4, 8])
 @pytest.mark.parametrize("batch", [3, 40])
 def test_wide_activation_rows(dev, bits, batch):
