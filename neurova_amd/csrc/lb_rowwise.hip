@@ -832,9 +832,13 @@ int launch_mm(const Params& p, int nw, int bits, hipStream_t st) {
 // kernel where the row does not fit LDS or the group is not a power of two of
 // units (g96 at 4 bits, K = 5120, N = 17408: 19.9 us, the matrix-core product
 // 20.9).  Everything else goes to the matrix-core product (ragged rows at that
-// size, 4 bits: 32.6 us against the general kernel's 132; a batch of 16 rows 21
-// against 196 us on four-row tiles of the fast kernel), except groups that are
-// neither a multiple of 32 columns nor the whole row: the general kernel.
+// size, 4 bits: 17.9 us against 25.5 on the fast kernel, where the rows are
+// dword-aligned, and 109 on the general one; a batch of 16 rows 21 against 196 us
+// on four-row tiles of the fast kernel), with two exceptions for the general
+// kernel: groups that are neither a multiple of 32 columns nor the whole row, and
+// code rows shorter than the product's 16-byte loads while the waves are few
+// enough to run together (7 columns, 8 bits: 1024 rows 4.4 against 6.0 us, batch 16
+// 5.2 against 9.1; 8192 rows, batch 16: 13.2 against 10.6).
 int launch(Params p, int nw, int bits, hipStream_t st) {
   const bool units = p.batch == 1 && p.cols % 32 == 0 && (p.packed_cols % 4 == 0) && lbh::aligned(p.q[0], 4) &&
                      (nw == 1 || lbh::aligned(p.q[1], 4)) && (p.group % 32 == 0) && lbh::aligned(p.x, 16);
@@ -850,7 +854,9 @@ int launch(Params p, int nw, int bits, hipStream_t st) {
     return nw == 1 ? launch_lds<1>(p, bits, st) : launch_lds<2>(p, bits, st);
   }
   if (units) return nw == 1 ? launch_fast<1>(p, bits, st) : launch_fast<2>(p, bits, st);
-  if (mm_takes(p)) return launch_mm(p, nw, bits, st);
+  const bool tiny = (p.cols * bits + 7) / 8 < 16 &&
+                    p.rows * ((p.batch + kMaxBatchTile - 1) / kMaxBatchTile) <= 80 * (int64_t)lbh::device_cus();
+  if (!tiny && mm_takes(p)) return launch_mm(p, nw, bits, st);
   if (p.batch <= 1) return nw == 1 ? launch_general<1, 1>(p, bits, st) : launch_general<2, 1>(p, bits, st);
   if (p.batch == 2) return launch_general<1, 2>(p, bits, st);
   return launch_general<1, kMaxBatchTile>(p, bits, st);

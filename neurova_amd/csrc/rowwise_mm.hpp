@@ -139,13 +139,32 @@ typedef u32x4 u32x4_any __attribute__((aligned(1)));
 __device__ __forceinline__ u32x4 load16(const void* base, uint32_t byte_off) {
   return *reinterpret_cast<const u32x4_any*>(reinterpret_cast<const char*>(base) + byte_off);
 }
-// Bytes at base + [0, 16) that lie before `limit`; the others are zero.
-__device__ __forceinline__ u32x4 load16_careful(const uint8_t* base, int limit) {
-  uint32_t v[4] = {0, 0, 0, 0};
+// Bytes [from, from + 16) of a row of `end` bytes, zeros past its end; nothing
+// outside the row is read.  One 16-byte load that ends inside the row, shifted
+// into place: the stage that ends a ragged row is a serial tail of one wave,
+// and sixteen byte loads a chunk there took half of a short launch (4 bits, one
+// row: K = 1144, N = 1024 9.8 -> 4.7 us, K = 2168, N = 4096 12.1 -> 5.5, K = 5240, N =
+// 17408 32.6 -> 17.8).
+__device__ __forceinline__ u32x4 load16_tail(const uint8_t* row, int from, int end) {
+  if (end < 16) {  // (uniform) the whole row is shorter than a load
+    uint32_t v[4] = {0, 0, 0, 0};
 #pragma unroll
-  for (int b = 0; b < 16; ++b)
-    if (b < limit) v[b >> 2] |= (uint32_t)base[b] << (8 * (b & 3));
-  return (u32x4){v[0], v[1], v[2], v[3]};
+    for (int b = 0; b < 16; ++b)
+      if (from + b < end) v[b >> 2] |= (uint32_t)row[from + b] << (8 * (b & 3));
+    return (u32x4){v[0], v[1], v[2], v[3]};
+  }
+  const int at = min(from, end - 16);
+  const u32x4 v = load16(row + at, 0);
+  const int bits = 8 * (from - at);
+  uint64_t lo = v[0] | ((uint64_t)v[1] << 32), hi = v[2] | ((uint64_t)v[3] << 32);
+  if (bits >= 64) {
+    lo = bits >= 128 ? 0 : hi >> (bits - 64);
+    hi = 0;
+  } else if (bits > 0) {
+    lo = (lo >> bits) | (hi << (64 - bits));
+    hi >>= bits;
+  }
+  return (u32x4){(uint32_t)lo, (uint32_t)(lo >> 32), (uint32_t)hi, (uint32_t)(hi >> 32)};
 }
 
 // The weight bytes of 16 NB rows of one stage, through LDS.  A load
@@ -192,8 +211,7 @@ struct Weights {
 #pragma unroll
     for (int t = 0; t < kLoads; ++t) {
       const int c = chunk(lane, t), row = c / BITS, seg = c - row * BITS;
-      const int from = stage * (16 * BITS) + 16 * seg;
-      r[t] = load16_careful(q + (int64_t)min(n0 + row, p.rows - 1) * p.packed_cols + from, row_bytes - from);
+      r[t] = load16_tail(q + (int64_t)min(n0 + row, p.rows - 1) * p.packed_cols, stage * (16 * BITS) + 16 * seg, row_bytes);
     }
   }
   __device__ __forceinline__ void store(char* lds, const u32x4 (&r)[kLoads]) const {
@@ -380,12 +398,11 @@ __global__ __launch_bounds__(W* kWave) void skinny_kernel(Params p) {
     wt.load_last(raw[0], p, q, plain, n0, lane);
     sc.load(sv[0], p, sp, plain, (p.cols - 1) / (kStageK / SPS));
 #pragma unroll
-    for (int t = 0; t < 4 * MB; ++t) {
-      const int k = plain * kStageK + 8 * nl;
-      xv[0][t] = load16_careful(
-          reinterpret_cast<const uint8_t*>(p.x + (int64_t)min(m0 + 4 * t + g, p.batch - 1) * p.x_stride + k),
-          2 * (p.cols - k));
-    }
+    for (int t = 0; t < 4 * MB; ++t)
+      if (4 * t < mrows)
+        xv[0][t] = load16_tail(
+            reinterpret_cast<const uint8_t*>(p.x + (int64_t)min(m0 + 4 * t + g, p.batch - 1) * p.x_stride),
+            2 * (plain * kStageK + 8 * nl), 2 * p.cols);
     stage_lds(0);
     compute(sv[0]);
   }
@@ -456,10 +473,9 @@ __global__ __launch_bounds__(kTileThreads, OCC) void tile_kernel(Params p) {
   auto load_last = [&](int stage) __attribute__((always_inline)) {
     wt.load_last(raw[0], p, q, stage, n0, lane);
     sc.load(sv[0], p, sp, stage, (p.cols - 1) / (kStageK / SPS));
-    const int k = stage * kStageK + 8 * xc;
 #pragma unroll
     for (int t = 0; t < MB; ++t)
-      xl[0][t] = load16_careful(reinterpret_cast<const uint8_t*>(p.x + xrow(t) + k), 2 * (p.cols - k));
+      xl[0][t] = load16_tail(reinterpret_cast<const uint8_t*>(p.x + xrow(t)), 2 * (stage * kStageK + 8 * xc), 2 * p.cols);
   };
   auto store_x = [&](int slot, int buf) __attribute__((always_inline)) {
 #pragma unroll

@@ -142,3 +142,51 @@ def test_staged_row_of_whole_units(dev, bits, rows, cols, group):
         q2 = torch.flip(q, (0,)).contiguous()
         a, b = lc.lowbit_gemv_pair(q, s, q2, s, xd, cols, group, bits)
         assert torch.equal(a, y) and torch.equal(b, lc.lowbit_gemv(q2, s, xd, cols, group, bits))
+
+
+@pytest.mark.parametrize("bits", [2, 3, 4, 5, 6, 7, 8])
+@pytest.mark.parametrize("batch", [1, 3, 40, 130])
+def test_every_tail_length(dev, bits, batch):
+    """Rows that end 1 to 127 columns into a stage of 128, with and without a whole
+    stage before: the end of a row is loaded by 16-byte words shifted into place,
+    rows below 16 bytes by bytes."""
+    for cols in [*range(1, 34), 63, 64, 65, 100, 119, 120, 121, 127, *range(129, 146), 191, 192, 200, 247, 249, 255]:
+        rows = 4100 if batch == 130 and cols == 249 else 21  # (four-wave tiles from 64 x 64 tiles for every CU)
+        print_case("mm-tail", bits, batch, cols)
+        _, packed, scales, x = O.make_rowwise_inputs(rows, cols, bits, 32, batch=batch, seed=bits + cols + batch)
+        got = _gemm(dev, packed, scales, x, cols, 32, bits)
+        _check(got, x, packed, scales, cols, 32, bits, f"b{bits} K={cols}")
+
+
+def test_tiny_rows_beyond_one_round_of_waves(dev):
+    """Code rows below 16 bytes: the byte-wise kernel up to 80 waves per CU, the
+    matrix-core product beyond."""
+    for batch, rows in ((4, 20480), (4, 20481), (5, 20481)):
+        print_case("mm-tiny", batch, rows)
+        _, packed, scales, x = O.make_rowwise_inputs(rows, 7, 8, 32, batch=batch, seed=batch)
+        _check(_gemm(dev, packed, scales, x, 7, 32, 8), x, packed, scales, 7, 32, 8, f"{batch}x{rows}")
+
+
+def test_ragged_rows_run_like_whole_ones(dev):
+    """A row that ends 120 columns into its last stage takes no longer than one that
+    fills it, beyond 1.4 times for the noise of either (1.8 times when the end of a
+    row was loaded by bytes)."""
+    import torch
+    from neurova_amd import capi
+
+    rows, bits, best = 17408, 4, {}
+    for cols in (5240, 5248):
+        pc = cols * bits // 8
+        q = torch.randint(0, 256, (rows, pc), dtype=torch.uint8, device=dev)
+        s = torch.full((rows, 41), 0.01, dtype=torch.float16, device=dev)
+        x, y = torch.ones((2, cols), dtype=torch.float16, device=dev), torch.empty((2, rows), dtype=torch.float16, device=dev)
+        print_case("mm-ragged-time", cols)
+        for _ in range(12):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            for _ in range(20):
+                assert capi.lowbit_gemm(q, s, x, y, cols, 128, bits) == 0
+            b.record()
+            torch.cuda.synchronize()
+            best[cols] = min(best.get(cols, 1e9), a.elapsed_time(b))
+    assert best[5240] < 1.4 * best[5248], best
