@@ -516,7 +516,14 @@ inline Plan make_plan(int64_t m, int64_t n, int64_t k, int64_t workspace_len, bo
     }
     // A round of 128-row tiles or more: they run whole, as many as fill the
     // resident slots a whole number of times, and the rest is split over K.
-    // (The argmax also takes this path with fewer tiles, 64 rows below M = 128.)
+    // The argmax takes this path with fewer tiles too (64 rows below M = 128): its
+    // keys need a tile's finished sums, so no second launch can make them, and
+    // stream-K, whose cut tiles each finish in one workgroup, is behind (g128: M =
+    // 2048, K = N = 5120 554 us against 405, K = 17408 734 against 592; M = 512, K =
+    // 4096, N = 32000 288 against 215; M = 1024, K = 2048, N = 8192 278 against 193).  So
+    // are more splits than the cost model's where they would give every CU a
+    // workgroup (K = 17408, N = 5120, 13 instead of 10: M = 17 35.2 us against 30.7, M =
+    // 32 38.3 against 33.3).
     pl.mb = m >= 128 ? 8 : (m > 32 ? 4 : 2);
     const int64_t bm = 16 * pl.mb;
     pl.n_mb = (int)((m + bm - 1) / bm);
@@ -692,7 +699,7 @@ int run(Variant var, const uint16_t* a, const int32_t* b, uint16_t* c, const uin
   hipLaunchKernelGGL((gemm::marlin_gemm_kernel<MBV, EPV, GV, SKV>), grid, dim3(gemm::kThreads), 0, st, p)
 #define LB_GM(MBV, EPV, GV)                                  \
   do {                                                       \
-    if constexpr (MBV == 8) {                                \
+    if constexpr (MBV == 8 && EPV == gemm::EPI_STORE) {      \
       if (pl.sk_wgs > 0) LB_GM_SK(MBV, EPV, GV, true);       \
       else LB_GM_SK(MBV, EPV, GV, false);                    \
     } else {                                                 \

@@ -185,3 +185,9 @@ def test_prefill_below_128_rows_is_not_streamk(L):
     for m, n, k, g, variant in itertools.product((33, 40, 64, 100, 127), (65536, 66560, 81920), (1024, 5120, 17408), (128, -1), (0, 1)):
         p = _plan(m, n, k, g, variant)
         assert p["form"] == "prefill" and (m > 64 or p["chunks_or_row_blocks"] < 8), f"m={m} n={n} k={k} g={g}: {p}"
+
+
+def test_argmax_prefill_is_not_streamk(L):
+    """The argmax runs whole tiles and split ones: stream-K has no argmax kernel."""
+    for m, n, k, g in itertools.product((128, 512, 1024, 2048), (5120, 8192, 32000, 65536), (1024, 5120, 17408), (128, -1)):
+        assert _plan(m, n, k, g, 2)["form"] == "prefill", (m, n, k, g)
