@@ -100,6 +100,10 @@ int lb_lowbit_row_dequant(const uint8_t* qweight, int64_t rows, int64_t packed_c
  *              sizes it N/128*16); left zero on return;
  * scratch:     device memory of at least lb_marlin_scratch_bytes() bytes
  *              (may be NULL when that is 0); contents need no initialisation.
+ *              With less, lb_marlin_gemm and lb_marlin_gemm_silu_packed run a
+ *              slower prefill plan where that needs no more than is given (with a
+ *              workspace of one entry it needs none); otherwise, as for every
+ *              other plan, LB_ERR_SCRATCH before anything is launched.
  * Requires N % 256 == 0 and K % 128 == 0; any M >= 0.
  */
 

@@ -169,6 +169,7 @@ struct Plan {
   int tail_tiles = 0;   // GEMM: tiles split over K ...
   int tail_splits = 1;  // ... this many ways
   bool two_pass = false; // GEMM: every tile is split and a second launch sums the partials
+  bool gate_in_tiles = false;  // GEMM, SiLU-gated: A gated by every tile, no activations in scratch
   int sk_wgs = 0;       // GEMM: > 0, the stream-K schedule over this many workgroups
   int64_t wgs = 0;      // GEMM workgroups
   size_t lds = 0;    // decode kernel dynamic LDS
@@ -349,7 +350,10 @@ inline Tiling direct_tiling(int64_t m, int64_t n, int64_t k, int64_t workspace_l
 
 // `gated`: the SiLU-gated projection;
 // `argmax`: the fused-argmax variant; `grouped`: group scales (else one per
-// column); `allow_mixed`: the mixed whole-K plan (grouped only) may be used.
+// column); `allow_mixed`: the mixed whole-K plan (grouped only) may be used;
+// `lean`: the prefill plan for a caller whose scratch is too small for the one
+// that is ahead: no gated activations, no splits summed by a second launch.
+// With a workspace too short for the split counters as well it needs no scratch.
 //
 // Which decode form (measured on the decode shapes of BASELINE.json): the direct
 // form where the tiles are narrow (the waves of a workgroup then share
@@ -372,7 +376,7 @@ constexpr int64_t kMixedDirectMaxM2 = 8;    // ... and with two whole-K tiles pe
 inline bool wave_a(int64_t m, int64_t k) { return m > 28 && k >= 4096; }
 
 inline Plan make_plan(int64_t m, int64_t n, int64_t k, int64_t workspace_len, bool gated, bool argmax = false,
-                      bool grouped = true, bool allow_mixed = true) {
+                      bool grouped = true, bool allow_mixed = true, bool lean = false) {
   Plan pl;
   pl.n_cg = (int)(n / 256);
   const int groups = (int)(k / 128);
@@ -465,11 +469,12 @@ inline Plan make_plan(int64_t m, int64_t n, int64_t k, int64_t workspace_len, bo
     if (direct && gated) pl.act_bytes = align_up((size_t)m * (size_t)k * 2);
   } else {
     pl.skinny = false;
-    if (gated) pl.act_bytes = align_up((size_t)m * (size_t)k * 2);
+    pl.gate_in_tiles = gated && lean;
+    if (gated && !lean) pl.act_bytes = align_up((size_t)m * (size_t)k * 2);
     pl.keys_bytes = align_up((size_t)m * (size_t)pl.n_cg * 8);
-    const int64_t slots = (int64_t)gemm::wgs_per_cu(8) * cus;      // of 128-row tiles
+    const int64_t slots = (int64_t)gemm::wgs_per_cu(8, gemm::A_PLAIN) * cus;  // of 128-row tiles
     const int64_t tiles8 = (int64_t)pl.n_cg * ((m + 127) / 128);
-    if (!argmax && tiles8 < slots) {
+    if (!argmax && !lean && tiles8 < slots) {
       // Less than one round of 128-row tiles: stream-K where it is ahead, else
       // the tile height and k split the cost model prefers.
       //
@@ -524,11 +529,13 @@ inline Plan make_plan(int64_t m, int64_t n, int64_t k, int64_t workspace_len, bo
     // are more splits than the cost model's where they would give every CU a
     // workgroup (K = 17408, N = 5120, 13 instead of 10: M = 17 35.2 us against 30.7, M =
     // 32 38.3 against 33.3).
-    pl.mb = m >= 128 ? 8 : (m > 32 ? 4 : 2);
+    // ``lean`` plans take it as well; tiles that gate their own A have 64 rows.
+    const int am = pl.gate_in_tiles ? gemm::A_SILU_PACKED : gemm::A_PLAIN;
+    pl.mb = m >= 128 && !pl.gate_in_tiles ? 8 : (m > 32 ? 4 : 2);
     const int64_t bm = 16 * pl.mb;
     pl.n_mb = (int)((m + bm - 1) / bm);
     const int64_t tiles = (int64_t)pl.n_cg * pl.n_mb;
-    const int64_t slots_mb = (int64_t)gemm::wgs_per_cu(pl.mb) * cus;
+    const int64_t slots_mb = (int64_t)gemm::wgs_per_cu(pl.mb, am) * cus;
     int64_t full = (tiles / slots_mb) * slots_mb;
     int64_t tail = tiles - full;
     int s = tail > 0 ? choose_tail_splits(tail, slots_mb, groups, pl.mb) : 1;
@@ -592,21 +599,17 @@ int run(Variant var, const uint16_t* a, const int32_t* b, uint16_t* c, const uin
   if (k * n / 2 >= (1LL << 32)) return LB_ERR_PROB_SHAPE;
   const bool gated = var == V_SILU || var == V_SILU_DONE;
   Plan pl = make_plan(m, n, k, workspace_len, gated, var == V_ARGMAX, grouped != 0);
-  // Without scratch for its partials a two-pass plan runs its tiles whole: a
-  // caller with a workspace too short for split counters could always call
-  // without scratch.
-  const size_t act_need = var == V_SILU ? pl.act_bytes : 0;
-  if (pl.two_pass && (!scratch || scratch_bytes < pl.partial_bytes + act_need)) {
-    pl.two_pass = false;
-    pl.full_tiles = pl.tail_tiles;
-    pl.tail_tiles = 0;
-    pl.tail_splits = 1;
-    pl.wgs = pl.full_tiles;
-    pl.partial_bytes = 0;
-  }
+  auto scratch_need = [&] {
+    return pl.partial_bytes + (var == V_ARGMAX ? pl.keys_bytes : 0) + (var == V_SILU ? pl.act_bytes : 0);
+  };
+  // Callers with less scratch than the two-launch splits or the gated
+  // activations take (header: the least a call needs)
+  const size_t usable = scratch && lbh::aligned(scratch, 16) ? scratch_bytes : 0;
+  if (!pl.skinny && (pl.two_pass || (var == V_SILU && pl.act_bytes > 0)) && usable < scratch_need())
+    pl = make_plan(m, n, k, workspace_len, gated, false, grouped != 0, true, true);
   if (var == V_SILU_DONE && !pl.skinny) return LB_ERR_ARG;  // decode batches only
   if (workspace_len < counters_needed(pl, var == V_ARGMAX)) return LB_ERR_WORKSPACE;
-  const size_t need = pl.partial_bytes + (var == V_ARGMAX ? pl.keys_bytes : 0) + act_need;
+  const size_t need = scratch_need();
   if (need > 0 && (!scratch || scratch_bytes < need)) return LB_ERR_SCRATCH;
   if (need > 0 && !lbh::aligned(scratch, 16)) return LB_ERR_ALIGN;
 
@@ -695,30 +698,33 @@ int run(Variant var, const uint16_t* a, const int32_t* b, uint16_t* c, const uin
   p.partial_bytes = (uint32_t)pl.partial_bytes;
   p.kp_total = (int)(k / 32); p.n_cg = pl.n_cg; p.n_mb = pl.n_mb;
   dim3 grid((unsigned)pl.wgs, 1, 1);
-#define LB_GM_SK(MBV, EPV, GV, SKV) \
-  hipLaunchKernelGGL((gemm::marlin_gemm_kernel<MBV, EPV, GV, SKV>), grid, dim3(gemm::kThreads), 0, st, p)
-#define LB_GM(MBV, EPV, GV)                                  \
-  do {                                                       \
-    if constexpr (MBV == 8 && EPV == gemm::EPI_STORE) {      \
-      if (pl.sk_wgs > 0) LB_GM_SK(MBV, EPV, GV, true);       \
-      else LB_GM_SK(MBV, EPV, GV, false);                    \
-    } else {                                                 \
-      LB_GM_SK(MBV, EPV, GV, false);                         \
-    }                                                        \
+#define LB_GM_SK(MBV, AMV, EPV, GV, SKV) \
+  hipLaunchKernelGGL((gemm::marlin_gemm_kernel<MBV, AMV, EPV, GV, SKV>), grid, dim3(gemm::kThreads), 0, st, p)
+#define LB_GM(MBV, AMV, EPV, GV)                                   \
+  do {                                                             \
+    if constexpr (MBV == 8 && EPV == gemm::EPI_STORE) {            \
+      if (pl.sk_wgs > 0) LB_GM_SK(MBV, AMV, EPV, GV, true);        \
+      else LB_GM_SK(MBV, AMV, EPV, GV, false);                     \
+    } else {                                                       \
+      LB_GM_SK(MBV, AMV, EPV, GV, false);                          \
+    }                                                              \
   } while (0)
-#define LB_GM_G(MBV, EPV)                      \
-  do {                                         \
-    if (grouped) LB_GM(MBV, EPV, true);        \
-    else LB_GM(MBV, EPV, false);               \
+#define LB_GM_G(MBV, AMV, EPV)                      \
+  do {                                              \
+    if (grouped) LB_GM(MBV, AMV, EPV, true);        \
+    else LB_GM(MBV, AMV, EPV, false);               \
   } while (0)
-#define LB_GM_MB(EPV)                      \
-  do {                                     \
-    if (pl.mb == 8) LB_GM_G(8, EPV);       \
-    else if (pl.mb == 4) LB_GM_G(4, EPV);  \
-    else LB_GM_G(2, EPV);                  \
+#define LB_GM_MB(EPV)                                     \
+  do {                                                    \
+    if (pl.mb == 8) LB_GM_G(8, gemm::A_PLAIN, EPV);       \
+    else if (pl.mb == 4) LB_GM_G(4, gemm::A_PLAIN, EPV);  \
+    else LB_GM_G(2, gemm::A_PLAIN, EPV);                  \
   } while (0)
   if (var == V_ARGMAX) LB_GM_MB(gemm::EPI_ARGMAX);
-  else LB_GM_MB(gemm::EPI_STORE);
+  else if (pl.gate_in_tiles) {  // 64-row tiles at most (make_plan)
+    if (pl.mb == 4) LB_GM_G(4, gemm::A_SILU_PACKED, gemm::EPI_STORE);
+    else LB_GM_G(2, gemm::A_SILU_PACKED, gemm::EPI_STORE);
+  } else LB_GM_MB(gemm::EPI_STORE);
   if (pl.two_pass) {
     const dim3 blocks((unsigned)(pl.tail_tiles * 4 * pl.mb), 1, 1);
 #define LB_RED(MBV, GV)                                                                                            \

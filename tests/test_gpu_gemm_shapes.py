@@ -134,3 +134,53 @@ def test_one_entry_workspace_without_scratch(dev, m, k, n):
     st = capi.marlin_gemm(to_dev(x, dev), to_dev(qw, dev), c, to_dev(sp, dev), ws, 128, None)
     assert st == 0, capi.status_string(st)
     assert_close_f16(to_np(c), O.marlin_gemm(x, qw, sp, 128), what=f"m={m} k={k} n={n}")
+
+
+@pytest.mark.parametrize("m,k,n", [(20, 256, 512), (33, 1024, 768), (64, 2048, 1280), (200, 1024, 2048), (1030, 256, 256)])
+@pytest.mark.parametrize("group", [128, -1])
+def test_silu_packed_prefill_without_scratch(dev, m, k, n, group):
+    """Without scratch for the gated activations every tile gates its own rows:
+    whole tiles with a one-entry workspace and no scratch, split ones with scratch
+    for the partials alone; the same outputs as with scratch up to the order of
+    the sums."""
+    import torch
+    from neurova_amd import capi
+
+    print_case("silu no scratch", m, k, n, group)
+    _, qw, _, sp, _ = O.make_marlin_inputs(m, k, n, group, seed=3400 + m)
+    mixed = np.random.default_rng(3400 + m).normal(0, 1, (m, 2 * k)).astype(np.float16)
+    a, b, s = to_dev(mixed, dev), to_dev(qw, dev), to_dev(sp, dev)
+    ref = O.marlin_gemm_silu_packed(mixed, qw, sp, k, group)
+    c, ws, sc = _buffers(dev, m, n, k, group)
+    act = -(-m * k * 2 // 256) * 256
+    assert capi.marlin_describe_plan(m, n, k, group, 1)["form"] == "prefill" and sc.numel() >= act
+    one = torch.zeros((1,), dtype=torch.int32, device=dev)
+    for workspace, scratch in ((one, None), (one, sc[1:]), (ws, sc[:act - 256])):
+        c.fill_(float("nan"))
+        st = capi.marlin_gemm_silu_packed(a, b, c, s, workspace, group, scratch)
+        if st == capi.LB_ERR_SCRATCH and workspace is ws:  # its partials need more than that
+            torch.cuda.synchronize()
+            assert bool(torch.isnan(c).all())
+            continue
+        assert st == 0, capi.status_string(st)
+        torch.cuda.synchronize()
+        assert int(ws.abs().sum()) == 0 and int(one.abs().sum()) == 0
+        assert_close_f16(to_np(c), ref, what=f"m={m} k={k} n={n} g={group}")
+
+
+def test_scratch_is_refused_as_missing_before_anything_runs(dev):
+    """A workspace that holds the split counters asks for splits: without scratch
+    for their partials the call is refused, plain and SiLU-gated."""
+    import torch
+    from neurova_amd import capi
+
+    m, k, n = 48, 2048, 2048
+    print_case("scratch refused", m, k, n)
+    _, qw, _, sp, x = O.make_marlin_inputs(m, k, n, 128, seed=3500)
+    c, ws, _ = _buffers(dev, m, n, k, 128)
+    b, s = to_dev(qw, dev), to_dev(sp, dev)
+    mixed = np.concatenate([x, x], axis=1)
+    assert capi.marlin_gemm(to_dev(x, dev), b, c, s, ws, 128, None) == capi.LB_ERR_SCRATCH
+    assert capi.marlin_gemm_silu_packed(to_dev(mixed, dev), b, c, s, ws, 128, None) == capi.LB_ERR_SCRATCH
+    torch.cuda.synchronize()
+    assert bool(torch.isnan(c).all()) and int(ws.abs().sum()) == 0
