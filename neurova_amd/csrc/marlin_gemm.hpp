@@ -126,11 +126,9 @@ __global__ __launch_bounds__(kThreads, wgs_per_cu(MB, AM)) void marlin_gemm_kern
   // writes position L & 15 of row L >> 4 and fetches the chunk that belongs
   // there.  A fragment -- A[r][32d + 16(g>>1) + 4(g&1) + {0..3}] ++ the same
   // + 8 -- is the (g&1) half of chunks 4d + 2(g>>1) and 4d + 2(g>>1) + 1: two
-  // 8-byte reads.  Register layout: entry (d, g, r) at ((4d + g) * kBlk + r),
-  // each (d, g) block padded by one entry so that the staging writes of one
-  // row, which go to different blocks, land in different banks.
+  // 8-byte reads.
   constexpr int kRowU4 = 16;
-  constexpr int kBlk = BM + 1;
+  constexpr int kBlk = BM + 1;  // gated: one (step, lane group) block of its layout
   constexpr int kBufU4 = kDma ? BM * kRowU4 : kSteps * 4 * kBlk;
   // two separate arrays (not one [2][...]): the compiler's wait placement then
   // tells the buffer-to-LDS DMA into one buffer from reads of the other, and
@@ -177,15 +175,8 @@ __global__ __launch_bounds__(kThreads, wgs_per_cu(MB, AM)) void marlin_gemm_kern
   const uint32_t psel = hsel ? 0x07030501u : 0x02060004u;
   const NibConsts nk = nib_consts();
 
-  // ---- A staging: items (row r, octet o) of 8 halves, r-major so that 16
-  // consecutive threads read one row's 256 contiguous bytes ----
-  constexpr int kAItems = BM * 16;
-  constexpr int kAPer = kAItems / kThreads;
-  static_assert(kAItems % kThreads == 0, "A staging items");
-  const int64_t a_row_halves = AM == A_SILU_PACKED ? 2 * (int64_t)p.k : (int64_t)p.k;
-  const __amdgpu_buffer_rsrc_t ra = buffer_of(p.a, (uint32_t)((int64_t)p.m * a_row_halves * 2));
-  uint4 areg[kDma ? 1 : kAPer];
-  uint4 ureg[AM == A_SILU_PACKED ? kAPer : 1];
+  // ---- A staging ----
+  const __amdgpu_buffer_rsrc_t ra = buffer_of(p.a, (uint32_t)((int64_t)p.m * p.k * (kDma ? 2 : 4)));
   const int wave_u = __builtin_amdgcn_readfirstlane(wave);
   constexpr int kRowsPerWave = BM / kWaves;
   // DMA source of lane L in a four-row instruction: tile row b + (L >> 4), b
@@ -219,57 +210,16 @@ __global__ __launch_bounds__(kThreads, wgs_per_cu(MB, AM)) void marlin_gemm_kern
   auto dma_a = [&](int stage, int buf) __attribute__((always_inline)) {
     dma_rows(stage, buf, 0, std::integral_constant<int, kRowsPerWave>{});
   };
-  auto load_a = [&](int stage) __attribute__((always_inline)) {
-    if (kDma) return;
-#pragma unroll
-    for (int t = 0; t < kAPer; ++t) {
-      const int item = tid + t * kThreads;
-      const int r = item >> 4, o = item & 15;
-      const uint32_t off = (uint32_t)(((int64_t)(m0 + r) * a_row_halves + (int64_t)stage * 128 + 8 * o) * 2);
-      areg[t] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(ra, off, 0, 0));
-      if (AM == A_SILU_PACKED)
-        ureg[t] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(ra, off + 2u * (uint32_t)p.k, 0, 0));
-    }
-  };
-  auto store_a = [&](int buf) __attribute__((always_inline)) {
-    if (kDma) return;
-#pragma unroll
-    for (int t = 0; t < kAPer; ++t) {
-      const int item = tid + t * kThreads;
-      const int r = item >> 4, o = item & 15;
-      uint4 w = areg[t];
-      if (AM == A_SILU_PACKED) {
-        const uint4 u = ureg[t];
-        const uint32_t gw[4] = {w.x, w.y, w.z, w.w};
-        const uint32_t uw[4] = {u.x, u.y, u.z, u.w};
-        uint32_t ov[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const float g0 = h2f((uint16_t)(gw[e] & 0xffffu)), g1 = h2f((uint16_t)(gw[e] >> 16));
-          const float u0 = h2f((uint16_t)(uw[e] & 0xffffu)), u1 = h2f((uint16_t)(uw[e] >> 16));
-          ov[e] = (uint32_t)f2h(silu(g0) * u0) | ((uint32_t)f2h(silu(g1) * u1) << 16);
-        }
-        w = make_uint4(ov[0], ov[1], ov[2], ov[3]);
-      }
-      // octet o = 4d + 2prow + half: halves 0..3 -> (d, g = 2prow), 4..7 -> (d, g = 2prow + 1)
-      const int d = o >> 2, pr = (o >> 1) & 1, half = o & 1;
-      uint2* dst0 = reinterpret_cast<uint2*>(&afr(buf)[(d * 4 + 2 * pr) * kBlk + r]) + half;
-      uint2* dst1 = reinterpret_cast<uint2*>(&afr(buf)[(d * 4 + 2 * pr + 1) * kBlk + r]) + half;
-      *dst0 = make_uint2(w.x, w.y);
-      *dst1 = make_uint2(w.z, w.w);
-    }
-  };
-
-  // ---- B ring: two stages of (4 slots + the group's scales) per lane ----
-  u32x4 bst[2][kSteps];
-  u32x4 sst[2];
-  auto load_b = [&](int slot, int stage) __attribute__((always_inline)) {
+  // ---- B: one stage of 4 slots and the group's scales per lane ----
+  u32x4 bst[kSteps];
+  u32x4 sst;
+  auto load_b = [&](int stage) __attribute__((always_inline)) {
 #pragma unroll
     for (int d = 0; d < kSteps; ++d)
-      bst[slot][d] = __builtin_bit_cast(
+      bst[d] = __builtin_bit_cast(
           u32x4, __builtin_amdgcn_raw_buffer_load_b128(rb, b_off, (uint32_t)(stage * 8 + 2 * d) * row_bytes, 0));
     if (GROUPED)
-      sst[slot] = __builtin_bit_cast(
+      sst = __builtin_bit_cast(
           u32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, s_off, (uint32_t)stage * (uint32_t)p.n * 2u, 0));
   };
 
@@ -279,48 +229,8 @@ __global__ __launch_bounds__(kThreads, wgs_per_cu(MB, AM)) void marlin_gemm_kern
 #pragma unroll
     for (int i = 0; i < MB; ++i) acc[j][i] = (f32x4){0.f, 0.f, 0.f, 0.f};
 
-  // dequantise step d of B slot `slot` into four fp16 fragments: exact fp16
-  // (q - 8) times the fp16 group scale, the rounding of the reference's __hmul2
-  auto dequant = [&](int slot, int d, const f16x2 (&sc)[4], f16x8 (&bf)[4]) __attribute__((always_inline)) {
-    const u32x4 own = bst[slot][d];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const uint32_t partner = (uint32_t)__builtin_amdgcn_mov_dpp((int)own[j], 0x128, 0xf, 0xf, false);  // row_ror:8
-      const uint32_t v0 = __builtin_amdgcn_perm(own[j], partner, psel);
-      const uint32_t v1 = v0 >> 8;
-      const f16x2 b0 = nib_lo_to_h2(v0, nk) * sc[j];
-      const f16x2 b1 = nib_lo_to_h2(v1, nk) * sc[j];
-      const f16x2 b2 = nib_hi_to_h2(v0, nk) * sc[j];
-      const f16x2 b3 = nib_hi_to_h2(v1, nk) * sc[j];
-      bf[j] = __builtin_bit_cast(f16x8, make_uint4(as_u32(b0), as_u32(b1), as_u32(b2), as_u32(b3)));
-    }
-  };
-  auto compute = [&](int buf, int slot, auto hook) __attribute__((always_inline)) {
-    f16x2 sc[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const uint32_t h = GROUPED ? ((sst[slot][j] >> (16 * hsel)) & 0xffffu) : 0x3c00u;  // fp16 1.0
-      sc[j] = as_h2(h | (h << 16));
-    }
-#pragma unroll
-    for (int d = 0; d < kSteps; ++d) {
-      f16x8 bfrag[4];
-      dequant(slot, d, sc, bfrag);
-      hook(d);
-      const uint4* abase = &afr(buf)[(d * 4 + g) * kBlk + (lane & 15)];
-#pragma unroll
-      for (int i = 0; i < MB; ++i) {
-        const f16x8 afrag = __builtin_bit_cast(f16x8, abase[16 * i]);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[j][i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(afrag, bfrag[j], acc[j][i], 0, 0, 0);
-      }
-      __builtin_amdgcn_sched_barrier(0);  // bound the registers live across steps
-    }
-  };
-
-  auto no_hook = [](int) __attribute__((always_inline)) {};
-
-  // ---- interleaved dequant (plain A) ----
+  // ---- interleaved dequant: exact fp16 (q - 8) times the fp16 group scale,
+  // the rounding of the reference's __hmul2 ----
   // One step's dequant split into 8 phases of one or two VALU instructions
   // per B word, so that step d + 1's dequant can be spread over the MFMAs of
   // step d (VALU instructions between a wave's MFMAs run in their shadow),
@@ -341,7 +251,7 @@ __global__ __launch_bounds__(kThreads, wgs_per_cu(MB, AM)) void marlin_gemm_kern
     const f16x2 k16 = {(f16)0.0625f, (f16)0.0625f}, k72 = {(f16)-72.0f, (f16)-72.0f};
     switch (ph) {
       case 0: {
-        const uint32_t own = bst[0][d][j];
+        const uint32_t own = bst[d][j];
         const uint32_t partner = (uint32_t)__builtin_amdgcn_mov_dpp((int)own, 0x128, 0xf, 0xf, false);  // row_ror:8
         q.v0[j] = __builtin_amdgcn_perm(own, partner, psel);
         pin_vgpr(q.v0[j]);
@@ -407,7 +317,7 @@ __global__ __launch_bounds__(kThreads, wgs_per_cu(MB, AM)) void marlin_gemm_kern
   auto scales_of = [&](f16x2 (&sc)[4]) __attribute__((always_inline)) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      const uint32_t h = GROUPED ? ((sst[0][j] >> (16 * hsel)) & 0xffffu) : 0x3c00u;  // fp16 1.0
+      const uint32_t h = GROUPED ? ((sst[j] >> (16 * hsel)) & 0xffffu) : 0x3c00u;  // fp16 1.0
       sc[j] = as_h2(h | (h << 16));
     }
   };
@@ -421,7 +331,7 @@ __global__ __launch_bounds__(kThreads, wgs_per_cu(MB, AM)) void marlin_gemm_kern
       for (int j = 0; j < 4; ++j) dq_word(q, 0, sc, ph, j);
     dq_pack(q, bcur);
   };
-  // One stage of plain-A compute.  On entry `bcur` holds step 0's B
+  // One stage of compute.  On entry `bcur` holds step 0's B
   // fragments and `sc` the stage's scales.  Step d's MFMAs (row block i's A
   // fragment read two blocks ahead) each carry a share of the dequant of step
   // d + 1 -- for the last step, of the next stage's step 0, whose slot and
@@ -485,14 +395,14 @@ __global__ __launch_bounds__(kThreads, wgs_per_cu(MB, AM)) void marlin_gemm_kern
     step(std::integral_constant<int, 3>{});
   };
 
-  // ---- pipeline (DMA A): the loads of stage s + 1 are issued during stage
+  // ---- pipeline: the loads of stage s + 1 are issued during stage
   // s -- A into the LDS buffer stage s - 1 used, each B slot into the
   // registers of the slot just dequantised.  A, the scales and B slots 0 and
   // 1 land before the barrier that ends stage s; slots 2 and 3 are waited for
   // where stage s + 1 dequantises them ----
   if (kDma && nst > 0) {
     dma_a(st0, 0);
-    load_b(0, st0);
+    load_b(st0);
     wait_vmcnt<0>();
     __syncthreads();
     f16x2 sc[4];
@@ -512,11 +422,11 @@ __global__ __launch_bounds__(kThreads, wgs_per_cu(MB, AM)) void marlin_gemm_kern
       // steps 0 .. 2 of the next stage.
       auto hook = [&](int d) __attribute__((always_inline)) {
         if (GROUPED && d == 0)
-          sst[0] = __builtin_bit_cast(
+          sst = __builtin_bit_cast(
               u32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, s_off, (uint32_t)nx * (uint32_t)p.n * 2u, 0));
         // step d's B slot is reloaded with stage s + 1's right after its
         // dequant, so one set of B registers serves both stages
-        bst[0][d] = __builtin_bit_cast(
+        bst[d] = __builtin_bit_cast(
             u32x4, __builtin_amdgcn_raw_buffer_load_b128(rb, b_off, (uint32_t)(nx * 8 + 2 * d) * row_bytes, 0));
         static_assert(kRowsPerWave % 2 == 0, "rows per half");
         if (d < 2) dma_rows(nx, c ^ 1, d * (kRowsPerWave / 2), std::integral_constant<int, kRowsPerWave / 2>{});
@@ -537,20 +447,108 @@ __global__ __launch_bounds__(kThreads, wgs_per_cu(MB, AM)) void marlin_gemm_kern
     // the last stage's extra DMA must land before the workgroup's LDS is released
     wait_vmcnt<0>();
   }
-  // ---- pipeline (register A): A one stage ahead, B two stages ahead ----
-  if (!kDma && nst > 0) {
-    load_a(st0);
-    load_b(0, st0);
-    if (nst > 1) load_b(1, st0 + 1);
-    store_a(0);
-    __syncthreads();
-    if (nst > 1) load_a(st0 + 1);
+
+  // ---- pipeline of the gated A: a stage of [g | u] into registers one stage
+  // ahead, gated and stored to LDS; B two stages ahead ----
+  if constexpr (!kDma) {
+    // items (row r, octet o) of 8 halves, r-major so that 16 consecutive threads
+    // read one row's 256 contiguous bytes
+    constexpr int kAItems = BM * 16;
+    constexpr int kAPer = kAItems / kThreads;
+    static_assert(kAItems % kThreads == 0, "A staging items");
+    uint4 areg[kAPer], ureg[kAPer];
+    auto load_a = [&](int stage) __attribute__((always_inline)) {
+#pragma unroll
+      for (int t = 0; t < kAPer; ++t) {
+        const int item = tid + t * kThreads;
+        const int r = item >> 4, o = item & 15;
+        const uint32_t off = (uint32_t)(((int64_t)(m0 + r) * 2 * p.k + (int64_t)stage * 128 + 8 * o) * 2);
+        areg[t] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(ra, off, 0, 0));
+        ureg[t] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(ra, off + 2u * (uint32_t)p.k, 0, 0));
+      }
+    };
+    // LDS layout: entry (d, g, r) at ((4d + g) * kBlk + r), each (d, g) block padded
+    // by one entry so that the stores of one row, which go to different blocks,
+    // land in different banks
+    auto store_a = [&](int buf) __attribute__((always_inline)) {
+#pragma unroll
+      for (int t = 0; t < kAPer; ++t) {
+        const int item = tid + t * kThreads;
+        const int r = item >> 4, o = item & 15;
+        const uint4 w = areg[t], u = ureg[t];
+        const uint32_t gw[4] = {w.x, w.y, w.z, w.w};
+        const uint32_t uw[4] = {u.x, u.y, u.z, u.w};
+        uint32_t ov[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float g0 = h2f((uint16_t)(gw[e] & 0xffffu)), g1 = h2f((uint16_t)(gw[e] >> 16));
+          const float u0 = h2f((uint16_t)(uw[e] & 0xffffu)), u1 = h2f((uint16_t)(uw[e] >> 16));
+          ov[e] = (uint32_t)f2h(silu(g0) * u0) | ((uint32_t)f2h(silu(g1) * u1) << 16);
+        }
+        // octet o = 4d + 2prow + half: halves 0..3 -> (d, g = 2prow), 4..7 -> (d, g = 2prow + 1)
+        const int d = o >> 2, pr = (o >> 1) & 1, half = o & 1;
+        uint2* dst0 = reinterpret_cast<uint2*>(&afr(buf)[(d * 4 + 2 * pr) * kBlk + r]) + half;
+        uint2* dst1 = reinterpret_cast<uint2*>(&afr(buf)[(d * 4 + 2 * pr + 1) * kBlk + r]) + half;
+        *dst0 = make_uint2(ov[0], ov[1]);
+        *dst1 = make_uint2(ov[2], ov[3]);
+      }
+    };
+    u32x4 bq[2][kSteps], bs[2];
+    auto load_b2 = [&](int slot, int stage) __attribute__((always_inline)) {
+#pragma unroll
+      for (int d = 0; d < kSteps; ++d)
+        bq[slot][d] = __builtin_bit_cast(
+            u32x4, __builtin_amdgcn_raw_buffer_load_b128(rb, b_off, (uint32_t)(stage * 8 + 2 * d) * row_bytes, 0));
+      if (GROUPED)
+        bs[slot] = __builtin_bit_cast(
+            u32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, s_off, (uint32_t)stage * (uint32_t)p.n * 2u, 0));
+    };
+    auto compute = [&](int buf, int slot) __attribute__((always_inline)) {
+      f16x2 sc[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const uint32_t h = GROUPED ? ((bs[slot][j] >> (16 * hsel)) & 0xffffu) : 0x3c00u;  // fp16 1.0
+        sc[j] = as_h2(h | (h << 16));
+      }
+#pragma unroll
+      for (int d = 0; d < kSteps; ++d) {
+        const u32x4 own = bq[slot][d];
+        f16x8 bf[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const uint32_t partner = (uint32_t)__builtin_amdgcn_mov_dpp((int)own[j], 0x128, 0xf, 0xf, false);  // row_ror:8
+          const uint32_t v0 = __builtin_amdgcn_perm(own[j], partner, psel);
+          const uint32_t v1 = v0 >> 8;
+          const f16x2 b0 = nib_lo_to_h2(v0, nk) * sc[j];
+          const f16x2 b1 = nib_lo_to_h2(v1, nk) * sc[j];
+          const f16x2 b2 = nib_hi_to_h2(v0, nk) * sc[j];
+          const f16x2 b3 = nib_hi_to_h2(v1, nk) * sc[j];
+          bf[j] = __builtin_bit_cast(f16x8, make_uint4(as_u32(b0), as_u32(b1), as_u32(b2), as_u32(b3)));
+        }
+        const uint4* abase = &afr(buf)[(d * 4 + g) * kBlk + (lane & 15)];
+#pragma unroll
+        for (int i = 0; i < MB; ++i) {
+          const f16x8 afrag = __builtin_bit_cast(f16x8, abase[16 * i]);
+#pragma unroll
+          for (int j = 0; j < 4; ++j) acc[j][i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(afrag, bf[j], acc[j][i], 0, 0, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);  // bound the registers live across steps
+      }
+    };
+    if (nst > 0) {
+      load_a(st0);
+      load_b2(0, st0);
+      if (nst > 1) load_b2(1, st0 + 1);
+      store_a(0);
+      __syncthreads();
+      if (nst > 1) load_a(st0 + 1);
+    }
     // Stage s uses LDS buffer and B slot s & 1; unrolled by two so that both
     // are compile-time constants (no indexed register access).
     auto stage = [&](int s, auto par) __attribute__((always_inline)) {
       constexpr int c = decltype(par)::value;
-      compute(c, c, no_hook);
-      if (s + 2 < nst) load_b(c, st0 + s + 2);
+      compute(c, c);
+      if (s + 2 < nst) load_b2(c, st0 + s + 2);
       if (s + 1 < nst) store_a(c ^ 1);  // buffer c ^ 1 was last read in stage s - 1
       __syncthreads();
       if (s + 2 < nst) load_a(st0 + s + 2);
