@@ -222,6 +222,7 @@ inline int choose_tail_splits(int64_t tail, int64_t slots, int groups, int mb) {
 // 200, N = 7168 37.6 -> 30.1 us.
 struct GemmShape {
   int mb = 8, splits = 1;
+  int64_t ns = 0;  // what the model prices it at
 };
 inline GemmShape choose_gemm_shape(int64_t m, int64_t n_cg, int groups, int64_t cus) {
   struct Height {
@@ -253,7 +254,41 @@ inline GemmShape choose_gemm_shape(int64_t m, int64_t n_cg, int groups, int64_t 
       }
     }
   }
+  best.ns = best_ns;
   return best;
+}
+
+// Stream-K (128-row tiles; every resident slot runs the same number of stages, a
+// tile is cut only where a workgroup's range ends) against the shape the model
+// above prefers, between half a round of tiles and a whole one.  Stream-K pays
+// about 40 us for the first loads and the cut tiles' partials and 3.0 us a stage,
+// more where the workgroups of one XCD (every eighth) start at many different k
+// offsets (64 / gcd(tiles, 64) of them: 8 or fewer are free).  Whole tiles, the
+// alternative nearly everywhere here, cost more a stage the more slots they fill;
+// up to one tile per CU they are never behind.  Both lines are fits to 150 launches
+// (12 M x N of 256 .. 448 tiles, K = 2048 .. 17408, both scale modes; rms error 4 and
+// 3 %), each repeated for a quarter of a second with bell-shaped codes: in short
+// bursts, and with codes of random bits, stream-K looks 7 to 10 % better than it is
+// in use.  It also draws more power, which the launches after it pay for (a layer of
+// 200 rows with stream-K for its gate/up projection, itself 2 % faster: 4 % slower),
+// so it has to be ahead by 7 %.
+//
+// The fixed conditions before (up to 52 % of a round; one scale per column and K
+// <= 2048; K > 8192 and whole sixty-fours of tiles) were up to 50 % off: g128, M =
+// 512, K = 8192, N = 17408 (272 tiles) 166 us whole, 144 as stream-K; M = 2048, K =
+// 17408, N = 4608 (288) 348 and 277; but M = 1024, K = 2048, N = 8448 (264) 48 and 64,
+// and with one scale per column M = 2048, K = 2048, N = 5120 (320) 51 and 73.
+// With one group a tile is never cut and the fit does not hold: stream-K takes 0.89
+// to 1.25 of the whole tiles' time there.
+inline bool streamk_ahead(int64_t tiles, int groups, int64_t slots, int64_t cus, const GemmShape& shape) {
+  if (groups == 1) return true;
+  if (tiles <= cus) return false;
+  int apart = 0;  // log2 of the different k offsets beyond eight
+  for (int64_t d = 8; d > 1 && tiles % d != 0; d /= 2) ++apart;
+  const int64_t sk = 40200 + tiles * groups * (3010 + 310 * apart) / slots;
+  const int64_t other = shape.mb == 8 && shape.splits == 1 ? 10600 + groups * (1728 + tiles * 1280 / slots)
+                                                           : 10600 + shape.ns * 9 / 10;
+  return sk * 100 < other * 93;
 }
 
 // Decode tiling with `cpw` chunks per workgroup: the k split count, or 0
@@ -351,9 +386,10 @@ inline Tiling direct_tiling(int64_t m, int64_t n, int64_t k, int64_t workspace_l
 // `gated`: the SiLU-gated projection;
 // `argmax`: the fused-argmax variant; `grouped`: group scales (else one per
 // column); `allow_mixed`: the mixed whole-K plan (grouped only) may be used;
-// `lean`: the prefill plan for a caller whose scratch is too small for the one
-// that is ahead: no gated activations, no splits summed by a second launch.
-// With a workspace too short for the split counters as well it needs no scratch.
+// `forms`: which prefill plans may be chosen, for a caller whose scratch is too
+// small for the one that is ahead.  F_LEAN: no stream-K, no gated activations, no
+// splits summed by a second launch; with a workspace too short for the split
+// counters as well it needs no scratch.
 //
 // Which decode form (measured on the decode shapes of BASELINE.json): the direct
 // form where the tiles are narrow (the waves of a workgroup then share
@@ -375,8 +411,10 @@ constexpr int64_t kMixedDirectMaxM2 = 8;    // ... and with two whole-K tiles pe
 // wave runs too few batches for it (M = 28, K = 2048, N = 3072 9.1 against 8.9 us).
 inline bool wave_a(int64_t m, int64_t k) { return m > 28 && k >= 4096; }
 
+enum Forms { F_ALL, F_NO_STREAMK, F_LEAN };
+
 inline Plan make_plan(int64_t m, int64_t n, int64_t k, int64_t workspace_len, bool gated, bool argmax = false,
-                      bool grouped = true, bool allow_mixed = true, bool lean = false) {
+                      bool grouped = true, bool allow_mixed = true, Forms forms = F_ALL) {
   Plan pl;
   pl.n_cg = (int)(n / 256);
   const int groups = (int)(k / 128);
@@ -469,34 +507,19 @@ inline Plan make_plan(int64_t m, int64_t n, int64_t k, int64_t workspace_len, bo
     if (direct && gated) pl.act_bytes = align_up((size_t)m * (size_t)k * 2);
   } else {
     pl.skinny = false;
-    pl.gate_in_tiles = gated && lean;
-    if (gated && !lean) pl.act_bytes = align_up((size_t)m * (size_t)k * 2);
+    pl.gate_in_tiles = gated && forms == F_LEAN;
+    if (gated && forms != F_LEAN) pl.act_bytes = align_up((size_t)m * (size_t)k * 2);
     pl.keys_bytes = align_up((size_t)m * (size_t)pl.n_cg * 8);
     const int64_t slots = (int64_t)gemm::wgs_per_cu(8, gemm::A_PLAIN) * cus;  // of 128-row tiles
     const int64_t tiles8 = (int64_t)pl.n_cg * ((m + 127) / 128);
-    if (!argmax && !lean && tiles8 < slots) {
-      // Less than one round of 128-row tiles: stream-K where it is ahead, else
-      // the tile height and k split the cost model prefers.
-      //
-      // Stream-K (every slot runs the same number of stages, a tile is cut
-      // only where a workgroup's range ends; two partial slots per workgroup)
-      // from half a round, and of that range only: just above half, where whole
-      // tiles would leave nearly half of the slots idle (264 tiles: K = 5120
-      // 103.6 us against 106.5, K = 17408 267-284 against 285; at K = 1024
-      // whole tiles would be ahead, 28 against 49 us); long K with tile counts
-      // of whole sixty-fours, whose workgroups on one XCD start at the same k
-      // offset (K = 17408: 320 tiles 301 us against 318 for three splits and
-      // 361 whole, but 300 tiles 335 against 300, 392 tiles 424 against 375
-      // whole); and one scale per column with a short K, which was not measured
-      // against the other forms.  Elsewhere whole tiles are ahead by up to a
-      // factor of two (M = 2048, K = 5120: N = 7168, 448 tiles, 124 against
-      // 144 us, N = 5120, 320 tiles, 110 against 118; K = 1024, N = 5120 31
-      // against 60 us).
+    if (!argmax && forms != F_LEAN && tiles8 < slots) {
+      // Less than one round of 128-row tiles: the tile height and k split the
+      // cost model prefers, or stream-K (two partial slots per workgroup)
+      const GemmShape g = choose_gemm_shape(m, pl.n_cg, groups, cus);
       const size_t sk_bytes = (size_t)2 * slots * 16 * 8 * gemm::kThreads * 4;
-      const bool sk = tiles8 * 100 <= slots * 52 || (!grouped && k <= 2048) ||
-                      (k > 8192 && tiles8 % 64 == 0 && tiles8 * 4 <= slots * 3);
-      if (sk && m >= 128 && tiles8 * 2 >= slots && workspace_len >= 1 + tiles8 && sk_bytes < ((size_t)1 << 31) &&
-          (int64_t)groups * tiles8 < ((int64_t)1 << 31)) {
+      if (forms == F_ALL && m >= 128 && tiles8 * 2 >= slots && workspace_len >= 1 + tiles8 &&
+          sk_bytes < ((size_t)1 << 31) && (int64_t)groups * tiles8 < ((int64_t)1 << 31) &&
+          streamk_ahead(tiles8, groups, slots, cus, g)) {
         pl.mb = 8;
         pl.n_mb = (int)((m + 127) / 128);
         pl.sk_wgs = (int)slots;
@@ -507,7 +530,6 @@ inline Plan make_plan(int64_t m, int64_t n, int64_t k, int64_t workspace_len, bo
         pl.partial_bytes = align_up(sk_bytes);
         return pl;
       }
-      const GemmShape g = choose_gemm_shape(m, pl.n_cg, groups, cus);
       pl.mb = g.mb;
       pl.n_mb = (int)((m + 16 * g.mb - 1) / (16 * g.mb));
       const int64_t tiles = (int64_t)pl.n_cg * pl.n_mb;
@@ -529,7 +551,7 @@ inline Plan make_plan(int64_t m, int64_t n, int64_t k, int64_t workspace_len, bo
     // are more splits than the cost model's where they would give every CU a
     // workgroup (K = 17408, N = 5120, 13 instead of 10: M = 17 35.2 us against 30.7, M =
     // 32 38.3 against 33.3).
-    // ``lean`` plans take it as well; tiles that gate their own A have 64 rows.
+    // F_LEAN plans take it as well; tiles that gate their own A have 64 rows.
     const int am = pl.gate_in_tiles ? gemm::A_SILU_PACKED : gemm::A_PLAIN;
     pl.mb = m >= 128 && !pl.gate_in_tiles ? 8 : (m > 32 ? 4 : 2);
     const int64_t bm = 16 * pl.mb;
@@ -602,11 +624,15 @@ int run(Variant var, const uint16_t* a, const int32_t* b, uint16_t* c, const uin
   auto scratch_need = [&] {
     return pl.partial_bytes + (var == V_ARGMAX ? pl.keys_bytes : 0) + (var == V_SILU ? pl.act_bytes : 0);
   };
-  // Callers with less scratch than the two-launch splits or the gated
-  // activations take (header: the least a call needs)
+  // Callers with less scratch than the plan that is ahead takes (header: the
+  // least a call needs).  Stream-K's best case, long K and a tile count of whole
+  // sixty-fours (K = 17408, 320 tiles 301 us, 361 whole), is asked for rather than
+  // run slower.
   const size_t usable = scratch && lbh::aligned(scratch, 16) ? scratch_bytes : 0;
+  if (pl.sk_wgs > 0 && usable < scratch_need() && !(k > 8192 && pl.tail_tiles % 64 == 0))
+    pl = make_plan(m, n, k, workspace_len, gated, false, grouped != 0, true, F_NO_STREAMK);
   if (!pl.skinny && (pl.two_pass || (var == V_SILU && pl.act_bytes > 0)) && usable < scratch_need())
-    pl = make_plan(m, n, k, workspace_len, gated, false, grouped != 0, true, true);
+    pl = make_plan(m, n, k, workspace_len, gated, false, grouped != 0, true, F_LEAN);
   if (var == V_SILU_DONE && !pl.skinny) return LB_ERR_ARG;  // decode batches only
   if (workspace_len < counters_needed(pl, var == V_ARGMAX)) return LB_ERR_WORKSPACE;
   const size_t need = scratch_need();

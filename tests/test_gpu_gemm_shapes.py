@@ -33,6 +33,8 @@ def _buffers(dev, m, n, k, g):
     (200, 5120, 5120, 128, None, True),
     (1000, 2304, 9216, 128, 8, False),  # 288 whole tiles, 96 rows of the last block missing
     (40, 256, 512, 128, None, None),    # two scale groups
+    (1000, 1024, 8448, 128, 8, False),  # few stages: whole tiles are ahead of stream-K from half a round on too
+    (1536, 2048, 8448, -1, 8, False),
 ])
 def test_shapes_vs_oracle(dev, m, k, n, group, height, split):
     import torch

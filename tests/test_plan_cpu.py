@@ -191,3 +191,18 @@ def test_argmax_prefill_is_not_streamk(L):
     """The argmax runs whole tiles and split ones: stream-K has no argmax kernel."""
     for m, n, k, g in itertools.product((128, 512, 1024, 2048), (5120, 8192, 32000, 65536), (1024, 5120, 17408), (128, -1)):
         assert _plan(m, n, k, g, 2)["form"] == "prefill", (m, n, k, g)
+
+
+@pytest.mark.parametrize("m,k,n,g,streamk_us,other_us", [
+    (512, 8192, 17408, 128, 143.5, 165.5), (200, 8192, 34816, -1, 132.1, 150.5), (1024, 17408, 8448, 128, 268.4, 341.3),
+    (2048, 17408, 4608, 128, 276.7, 347.8), (2048, 8192, 4608, -1, 138.1, 160.1), (2048, 17408, 5120, 128, 304.0, 354.0),
+    (2048, 17408, 5120, -1, 284.1, 334.3), (2048, 13824, 5120, 128, 247.9, 283.1), (1500, 17408, 7168, 128, 329.3, 356.7),
+    (1024, 2048, 8448, 128, 63.7, 48.1), (1024, 4096, 8448, -1, 88.9, 86.4), (2048, 2048, 5120, -1, 72.8, 50.8),
+    (2048, 4096, 5120, 128, 105.1, 90.2), (2048, 5120, 5120, 128, 120.7, 109.9), (1024, 5120, 14336, 128, 147.0, 125.4),
+    (1024, 2048, 14336, -1, 79.8, 55.2), (2048, 2048, 4096, 128, 54.9, 37.0), (2048, 5120, 4096, -1, 84.1, 76.3),
+    (1900, 5120, 5632, 128, 132.6, 111.2), (1900, 8192, 5632, -1, 193.7, 164.1), (700, 2048, 16384, -1, 70.3, 51.7),
+])
+def test_streamk_where_it_measured_ahead(L, m, k, n, g, streamk_us, other_us):
+    """Between half a round of 128-row tiles and a whole one the planner takes the
+    schedule that measured faster, by 7 % or more (256 compute units)."""
+    assert (_plan(m, n, k, g)["form"] == "prefill-streamk") == (streamk_us < other_us)
