@@ -124,11 +124,10 @@ size_t lb_marlin_scratch_bytes(int64_t prob_m, int64_t prob_n, int64_t prob_k, i
  *       tail tiles; stream-K: 1;
  *   [3] decode: 16-row MFMA blocks; split-tail: whole tiles; stream-K: 0;
  *   [4] workgroups; [5] dynamic LDS bytes per workgroup; [6] scratch bytes;
- *   [7] workspace entries used; [8] kernel launches (forms 1 and 2 of variant 1:
- *   2, the gated activations are formed in a launch of their own; forms 3 and
- *   4 count the GEMM's launch alone: variant 1 has that one before it, and a
- *   form 3 plan with every tile split, [2] > 1 and [3] = 0, one that sums the
- *   partials after it); [9] compute units planned for.
+ *   [7] workspace entries used; [8] kernel launches: the product's, one before
+ *   it for variant 1 on every form but 0 (the gated activations), and one after
+ *   it where all tiles of form 3 are split ([2] > 1 and [3] = 0 of variants 0
+ *   and 1: the sums of the partials); [9] compute units planned for.
  * Returns LB_OK, or the status the entry point would return for the shape. */
 int lb_marlin_describe_plan(int64_t prob_m, int64_t prob_n, int64_t prob_k, int64_t groupsize, int32_t variant,
                             int64_t workspace_len, int64_t* out);
@@ -213,7 +212,8 @@ int lb_marlin_mlp_fused(const uint16_t* x, const int32_t* gate_up_qweight, const
  * the process ends; problems whose plan needs more return
  * LB_ERR_NOALLOC_LIMIT before anything is launched (every decode shape up to
  * M = 64 of the BASELINE.json projections and of the reference's published
- * ones, lm_head 5120 -> 248320 included, fits; M = 2048 prefill does not).  All
+ * ones, lm_head 5120 -> 248320 included, fits; prefill plans with more split
+ * tiles than that, and the stream-K plan of M = 2048, K = 17408, N = 5120, do not).  All
  * calls on one GPU share that array: calls that overlap (other streams) race
  * and must be serialised by the caller.  Same arguments, workspace contract
  * and results as lb_marlin_gemm. */

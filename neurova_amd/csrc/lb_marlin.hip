@@ -840,7 +840,7 @@ extern "C" int lb_marlin_describe_plan(int64_t prob_m, int64_t prob_n, int64_t p
   }
   out[6] = (int64_t)(pl.partial_bytes + (argmax ? pl.keys_bytes : 0) + (gated ? pl.act_bytes : 0));
   out[7] = marlin::counters_needed(pl, argmax);
-  out[8] = (gated && pl.direct) ? 2 : 1;
+  out[8] = 1 + (gated && pl.act_bytes > 0 ? 1 : 0) + (pl.two_pass ? 1 : 0);
   out[9] = marlin::device_cus();
   return LB_OK;
 }
