@@ -107,7 +107,8 @@ int lb_lowbit_row_dequant(const uint8_t* qweight, int64_t rows, int64_t packed_c
  * Requires N % 256 == 0 and K % 128 == 0; any M >= 0.
  */
 
-/* Bytes of scratch the Marlin entry points need for this problem. */
+/* Bytes of scratch that cover every Marlin entry point at this size, either
+ * scale mode and any workspace (lb_marlin_describe_plan tells one call's need). */
 size_t lb_marlin_scratch_bytes(int64_t prob_m, int64_t prob_n, int64_t prob_k, int64_t groupsize);
 
 /* The plan a Marlin entry point makes for this problem (no counterpart in the

@@ -207,8 +207,13 @@ OpScratch op_scratch(size_t bytes, const torch::Tensor& like) {
   return r;
 }
 
-OpScratch scratch_for(int64_t m, int64_t n, int64_t k, int64_t g, const torch::Tensor& like) {
-  return op_scratch(lb_marlin_scratch_bytes(m, n, k, g), like);
+// What this call's own plan needs (lb_marlin_scratch_bytes covers every variant
+// and both scale modes, the gated activations [M][K] among them).  variant: 0
+// plain, 1 SiLU-gated, 2 argmax.
+OpScratch scratch_for(int variant, const MarlinShape& sh, const torch::Tensor& workspace, const torch::Tensor& like) {
+  int64_t plan[10];
+  const int err = lb_marlin_describe_plan(sh.m, sh.n, sh.k, sh.group, variant, workspace.numel(), plan);
+  return op_scratch(err == LB_OK ? (size_t)plan[6] : 0, like);  // a refused shape is refused by the call
 }
 
 void run_lowbit_marlin_gemm(torch::Tensor qweight, torch::Tensor scales, torch::Tensor x, torch::Tensor out,
@@ -223,7 +228,7 @@ void run_lowbit_marlin_gemm(torch::Tensor qweight, torch::Tensor scales, torch::
   const MarlinShape sh = check_marlin_common(qweight, scales, out, workspace, x.size(0), cols, group_size,
                                              "marlin out shape mismatch");
   const c10::DeviceGuard guard(x.device());
-  auto scratch = scratch_for(sh.m, sh.n, sh.k, sh.group, x);
+  auto scratch = scratch_for(0, sh, workspace, x);
   const int err = lb_marlin_gemm(h16(x), qweight.data_ptr<int32_t>(), h16m(out), h16(scales), sh.m, sh.n, sh.k,
                                  workspace.data_ptr<int32_t>(), workspace.numel(), sh.group, scratch.ptr,
                                  scratch.bytes, stream_of(x));
@@ -259,7 +264,7 @@ void lowbit_marlin_gemm_silu_packed_out(torch::Tensor qweight, torch::Tensor sca
   const MarlinShape sh = check_marlin_common(qweight, scales, out, workspace, mixed.size(0), cols, group_size,
                                              "marlin out shape mismatch");
   const c10::DeviceGuard guard(mixed.device());
-  auto scratch = scratch_for(sh.m, sh.n, sh.k, sh.group, mixed);
+  auto scratch = scratch_for(1, sh, workspace, mixed);
   const int err = lb_marlin_gemm_silu_packed(h16(mixed), qweight.data_ptr<int32_t>(), h16m(out), h16(scales), sh.m,
                                              sh.n, sh.k, workspace.data_ptr<int32_t>(), workspace.numel(), sh.group,
                                              scratch.ptr, scratch.bytes, stream_of(mixed));
@@ -291,7 +296,7 @@ void lowbit_marlin_gemm_argmax_out(torch::Tensor qweight, torch::Tensor scales, 
   TORCH_CHECK(argmax_sync.dim() == 1 && argmax_sync.numel() >= 2, "argmax_sync must be [2]");
   TORCH_CHECK(argmax_epoch > 0, "argmax_epoch must be positive");
   const c10::DeviceGuard guard(x.device());
-  auto scratch = scratch_for(sh.m, sh.n, sh.k, sh.group, x);
+  auto scratch = scratch_for(2, sh, workspace, x);
   const int err = lb_marlin_gemm_argmax(h16(x), qweight.data_ptr<int32_t>(), h16(scales), sh.m, sh.n, sh.k,
                                         workspace.data_ptr<int32_t>(), workspace.numel(), sh.group,
                                         argmax_state.data_ptr<int64_t>(), argmax_out.data_ptr<int64_t>(),

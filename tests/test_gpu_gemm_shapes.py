@@ -186,3 +186,36 @@ def test_scratch_is_refused_as_missing_before_anything_runs(dev):
     assert capi.marlin_gemm_silu_packed(to_dev(mixed, dev), b, c, s, ws, 128, None) == capi.LB_ERR_SCRATCH
     torch.cuda.synchronize()
     assert bool(torch.isnan(c).all()) and int(ws.abs().sum()) == 0
+
+
+@pytest.mark.parametrize("op,m,k,n", [("plain", 2048, 17408, 256), ("plain", 1024, 1024, 4096), ("gated", 300, 2048, 1024),
+                                      ("argmax", 40, 1024, 2048), ("plain", 4, 5120, 5120)])
+def test_op_scratch_is_its_plans_own(dev, op, m, k, n):
+    """The torch ops keep scratch for the plans they run, in whole MiB a stream: a
+    plain product none for gated activations."""
+    import torch
+    import langburst_cuda as lc
+    from neurova_amd import capi
+
+    need = capi.marlin_describe_plan(m, n, k, 128, ("plain", "gated", "argmax").index(op))["scratch_bytes"]
+    print_case("op scratch", op, m, k, n, need)
+    q = torch.zeros((k // 16, 2 * n), dtype=torch.int32, device=dev)
+    s = torch.ones((k // 128, n), dtype=torch.float16, device=dev)
+    x = torch.zeros((m, k * (2 if op == "gated" else 1)), dtype=torch.float16, device=dev)
+    out = torch.empty((m, n), dtype=torch.float16, device=dev)
+    ws = torch.zeros((n // 128 * 16,), dtype=torch.int32, device=dev)
+    best, state = (torch.zeros((m,), dtype=torch.int64, device=dev) for _ in range(2))
+    sync = torch.zeros((2,), dtype=torch.int32, device=dev)
+    side = torch.cuda.Stream()  # scratch is kept per stream
+    torch.cuda.synchronize()
+    with torch.cuda.stream(side):
+        before = torch.cuda.memory_allocated(dev)
+        if op == "plain":
+            lc.lowbit_marlin_gemm_out(q, s, x, out, ws, k, 128)
+        elif op == "gated":
+            lc.lowbit_marlin_gemm_silu_packed_out(q, s, x, out, ws, k, 128)
+        else:
+            lc.lowbit_marlin_gemm_argmax_out(q, s, x, out, ws, state, best, sync, 1, k, 128)
+        kept = torch.cuda.memory_allocated(dev) - before
+    torch.cuda.synchronize()
+    assert kept <= -(-need // 2 ** 20) * 2 ** 20, (kept, need)
