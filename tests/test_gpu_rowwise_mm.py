@@ -50,8 +50,8 @@ def test_edges_vs_oracle(dev, bits, rows, cols, group, batch):
     _check(_gemm(dev, packed, scales, x, cols, group, bits), x, packed, scales, cols, group, bits, f"b{bits}")
 
 
-# (batch, rows): one of each launch form on 256 compute units -- output blocks of 16 and 32
-# rows, one, two and four row blocks, eight and four waves, and the four tile shapes
+# (batch, rows): output blocks of 16 and 32 rows, one, two and four row blocks, eight and four
+# waves, and the four tile shapes, at rows of up to three stages
 @pytest.mark.parametrize("batch,rows", [(16, 4100), (32, 4100), (32, 8200), (64, 4100), (130, 4100), (65, 16400),
                                         (130, 5504), (512, 6144), (512, 12300)])
 @pytest.mark.parametrize("bits,cols,group", [(2, 256, 64), (3, 300, 32), (4, 384, 128), (7, 270, 32), (8, 256, 128)])
@@ -59,6 +59,42 @@ def test_launch_forms_vs_oracle(dev, batch, rows, bits, cols, group):
     print_case("mm-form", batch, rows, bits, cols, group)
     _, packed, scales, x = O.make_rowwise_inputs(rows, cols, bits, group, batch=batch, seed=bits + rows + batch)
     _check(_gemm(dev, packed, scales, x, cols, group, bits), x, packed, scales, cols, group, bits, f"{batch}x{rows}")
+
+
+# (batch, rows) for every launch form on 256 compute units, in the order of
+# launch_sps (lb_rowwise_mm.hip): up to 16 rows -- 48, 32 (two stages in flight, then
+# one) and 16 output rows a workgroup; up to 32 -- 48 and 32 rows on four waves, 32
+# and 16 on eight, blocks of 16; split K above -- four row blocks on eight and on four
+# waves, two row blocks of 16 output rows; the four tile shapes
+_FORMS = [(16, 16400), (8, 4100), (16, 8200), (16, 2100), (32, 17408), (32, 8300), (32, 4100), (32, 2100), (32, 1100),
+          (64, 4100), (130, 4100), (48, 1100), (512, 12300), (512, 6144), (65, 16400), (130, 5504)]
+
+
+@pytest.mark.parametrize("bits", [2, 3, 4, 5, 6, 7, 8])
+@pytest.mark.parametrize("group", [32, 64, 128])
+def test_pipelines_vs_oracle(dev, bits, group):
+    """Every launch form at every width and scale layout with several stages a wave
+    (25 whole ones over four or eight waves, or for one tile) and a ragged end:
+    slots issued again, LDS rows overwritten stage after stage.  Output rows of the
+    first and last workgroups and some between are checked."""
+    import torch
+    from neurova_amd import capi
+
+    cols = 25 * 128 + 7
+    gen = torch.Generator(device=dev)
+    gen.manual_seed(bits * 1000 + group)
+    for batch, rows in _FORMS:
+        print_case("mm-pipeline", bits, group, batch, rows)
+        q = torch.randint(0, 256, (rows, (cols * bits + 7) // 8), dtype=torch.uint8, device=dev, generator=gen)
+        s = (torch.rand((rows, -(-cols // group)), device=dev, generator=gen) * 0.01 + 1e-3).half()
+        x = torch.randn((batch, cols), device=dev, generator=gen).half()
+        y = torch.full((batch, rows), float("nan"), dtype=torch.float16, device=dev)
+        assert capi.lowbit_gemm(q, s, x, y, cols, group, bits) == 0
+        assert bool(torch.isfinite(y).all())
+        pick = np.unique(np.concatenate([np.arange(0, 49, 3), [63, 64, 127, 128, 255, 256], np.linspace(300, rows - 50, 9).astype(int),
+                                         np.arange(rows - 49, rows, 4), [rows - 1]]))
+        idx = torch.from_numpy(pick).to(dev)
+        _check(to_np(y[:, idx]), to_np(x), to_np(q[idx]), to_np(s[idx]), cols, group, bits, f"b{bits} g{group} {batch}x{rows}")
 
 
 @pytest.mark.parametrize("batch", [8, 9, 17, 32])
