@@ -406,9 +406,11 @@ constexpr int64_t kMixedMaxM = 4;      // rows with the A slice staged (measured
 constexpr int64_t kMixedDirectMaxM = 32;    // rows with A loaded per step, one whole-K tile per CU
 constexpr int64_t kMixedDirectMaxM2 = 8;    // ... and with two whole-K tiles per CU
 
-// Where the direct form's A goes through the waves' own LDS (skinny::A_WAVE): at
-// M = 28 the two are even at K = 5120, N = 5120 (11.8 us) and with a short K a
-// wave runs too few batches for it (M = 28, K = 2048, N = 3072 9.1 against 8.9 us).
+// Where the direct form's A goes through the waves' own LDS (skinny::A_WAVE): ahead
+// on every projection from 29 rows (figures there); at 24 to 28 ahead on wide ones,
+// even or behind on narrow ones (M = 24: K = 5120, N = 14336 16.2 -> 15.9 us, N = 5120
+// 11.1 -> 11.3), and with a short K a wave runs too few batches for it (K = 2048, N =
+// 3072: M = 28 8.9 against 9.0 us, M = 32 even).
 inline bool wave_a(int64_t m, int64_t k) { return m > 28 && k >= 4096; }
 
 enum Forms { F_ALL, F_NO_STREAMK, F_LEAN };

@@ -28,9 +28,9 @@ int launch_tile(const Params& p, hipStream_t st) {
 // 17408 and 17408 x 5120 (times below: 4 bits, g128):
 //   up to 16 rows: 32 output rows per workgroup (M = 16, N = 5120: 24 us, 16
 //     rows 34 us, 64 rows 38 us), 16 where that leaves half the CUs idle.  One
-//     stage in flight per wave: with two the registers leave room for one
-//     workgroup per CU instead of two (M = 16, N = 17408: 25.8 us against 22.5,
-//     8 bits 32.3 against 29.8).  Two in flight where there is one workgroup per
+//     stage in flight per wave: with two the registers (130 at first, 128 now) leave
+//     little or no room for a second workgroup on a CU (M = 16, N = 17408: 24.7 us
+//     against 22.8, 8 bits 32.3 against 29.8).  Two in flight where there is one workgroup per
 //     CU at most anyway, few rows and few bits (K = 17408, N = 5120, M = 6: 19.8
 //     against 20.2 us; 2 bits 16.8 against 18.7 at M = 4, even at 16).
 //     More than two workgroups of 32 rows per CU: 48 rows from M = 9 on, up to
@@ -48,6 +48,12 @@ int launch_tile(const Params& p, hipStream_t st) {
 //   else the largest tile that gives 1.5 workgroups per CU (N = 17408: M = 384
 //     102 us on 64 x 256, M = 256 79 us on 64 x 128 against 99, M = 128 51 us on
 //     32 x 128 against 56).
+// At 5, 6 and 7 bits (checked afterwards, g128, M = 4..384, the two shapes and N =
+// 34816) the same rules give the fastest form or one within 5 % of it, except: K =
+// 17408, N = 5120, M = 128, where eight waves (5 bits, 85 us against 122) or 64 x 64
+// tiles (6 and 7 bits, 107 and 111 against 120 and 126) are ahead, and N = 34816, where
+// 48 rows up to M = 16 (5 bits 38.6 against 42.9), 64 x 64 tiles at M = 64 (72 against
+// 81) and 64 x 128 at M = 384 (220 against 246) are.
 template <int SPS>
 int launch_sps(const Params& p, int mats, hipStream_t st) {
   const int64_t cus = lbh::device_cus();

@@ -471,9 +471,9 @@ __device__ __forceinline__ bool skinny_tile(const Params p, const int cg, const 
   // the wave's own LDS rows: halves 4 gq .. + 3 and 8 + 4 gq .. + 3 of a k16 row
   // are two 8-byte reads 16 bytes apart, which the padding spreads over all
   // banks.  No barrier: a wave reads what it stored.  The LDS round trip pays
-  // near the full 32 rows (M = 32: K = 5120, N = 14336 19.5 -> 17.3 us, N = 7168
-  // 14.8 -> 13.9, K = 17408, N = 5120 23.8 -> 22.1; M = 24 even; M = 16 and below
-  // up to 10 % slower, also where only two workgroups per CU were asked for).
+  // near the full 32 rows (M = 32: K = 5120, N = 14336 18.5 -> 16.0 us, N = 7168
+  // 14.7 -> 13.4, N = 5120 12.1 -> 11.7, K = 17408, N = 5120 22.2 -> 20.1; even from M
+  // = 24 on the wide projections to 28 on the narrow ones; M = 17 4 to 8 % slower).
   char* const wa = reinterpret_cast<char*>(smem) + wave * (kRows * kWaveRowBytes);
   uint32_t aoff[4 * MR];
   if constexpr (kWaveA) {
