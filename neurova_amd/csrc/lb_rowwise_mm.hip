@@ -35,7 +35,12 @@ int launch_tile(const Params& p, hipStream_t st) {
 //     against 20.2 us; 2 bits 16.8 against 18.7 at M = 4, even at 16).
 //     More than two workgroups of 32 rows per CU: 48 rows from M = 9 on, up to
 //     4 bits (M = 16: N = 17408 22.5 -> 21.0 us, N = 34816 36.0 -> 31.4; M = 3
-//     16.3 against 17.2; 5 bits 26.0 against 26.5);
+//     16.3 against 17.2; 5 bits 26.0 against 26.5).
+//     One (ragged) row, 16 output rows a workgroup on half the CUs at most: a
+//     wave's chain of stages is the launch, so sixteen waves take it from K = 8192
+//     on (2..8 bits, K = 17400: N = 2048 11.2..13.8 -> 8.7..11.7 us, N = 48 8.6..12.4
+//     -> 7.6..10.8; K = 8184 0.99 to 1.14 times as fast, K = 4088 0.85 to 0.98; with 4
+//     activation rows 0.95 at K = 12280, with 16 0.93 at K = 17400);
 //   17 to 32: two blocks of 16, eight waves and 32 rows (M = 32, N = 5120: 31
 //     us; 16 rows 46, four waves 45).  It is one workgroup per CU by its LDS, so
 //     with more than one for each four waves run (N = 14336 21.5 -> 20.5 us, K =
@@ -68,6 +73,7 @@ int launch_sps(const Params& p, int mats, hipStream_t st) {
           return launch_skinny<SPS, 1, 2, 8, 2>(p, mats, st);
     }
     if (2 * wgs(1, 32) >= cus) return launch_skinny<SPS, 1, 2, 8, 1>(p, mats, st);
+    if (p.batch == 1 && 2 * wgs(1, 16) <= cus && p.cols >= 8192) return launch_skinny<SPS, 1, 1, 16, 2>(p, mats, st);
     return launch_skinny<SPS, 1, 1, 8, 2>(p, mats, st);
   }
   const bool narrow = wgs(4, 64) < cus;

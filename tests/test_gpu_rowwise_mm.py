@@ -226,3 +226,56 @@ def test_ragged_rows_run_like_whole_ones(dev):
             torch.cuda.synchronize()
             best[cols] = min(best.get(cols, 1e9), a.elapsed_time(b))
     assert best[5240] < 1.4 * best[5248], best
+
+
+@pytest.mark.parametrize("bits", [2, 3, 4, 5, 6, 7, 8])
+@pytest.mark.parametrize("cols,group", [(8191, 128), (8193, 128), (8194, 64), (8290, 32), (12280, 128), (17400, 32), (17407, 64)])
+def test_long_ragged_row_of_few_outputs(dev, bits, cols, group):
+    """One row from K = 8192 on over blocks of 16 output rows on at most half of 256
+    compute units (2048 output rows): sixteen waves share it, some with one stage more
+    than others, and the ragged end is the next wave's; eight waves on either side."""
+    import langburst_cuda as lc
+    import torch
+
+    for rows in (1, 17, 2048, 2049):
+        if rows > 17 and cols != 8290:
+            continue
+        print_case("mm-long-row", bits, rows, cols, group)
+        _, packed, scales, x = O.make_rowwise_inputs(rows, cols, bits, group, batch=1, seed=bits + cols)
+        got = _gemm(dev, packed, scales, x, cols, group, bits)
+        _check(got, x, packed, scales, cols, group, bits, f"b{bits} {rows}x{cols}")
+        # two matrices in one launch: half the output rows each up to the same line
+        q, s, xd = to_dev(packed, dev), to_dev(scales, dev), to_dev(x[0], dev)
+        q2 = torch.flip(q, (0,)).contiguous()
+        a, b = lc.lowbit_gemv_pair(q, s, q2, s, xd, cols, group, bits)
+        _check(to_np(a)[None], x, packed, scales, cols, group, bits, "pair 0")
+        _check(to_np(b)[None], x, packed[::-1].copy(), scales, cols, group, bits, "pair 1")
+
+
+def test_long_ragged_row_of_few_outputs_time(dev):
+    """Sixteen waves on such a row: no slower than 0.93 of the same row in a batch of
+    two, which takes eight (measured 0.76 to 0.8)."""
+    import torch
+    from neurova_amd import capi
+
+    rows, bits, cols, best = 2048, 4, 17400, {}
+    q = torch.randint(0, 256, (rows, cols * bits // 8), dtype=torch.uint8, device=dev)
+    s = torch.full((rows, -(-cols // 128)), 0.01, dtype=torch.float16, device=dev)
+    for batch in (1, 2):
+        x = torch.ones((batch, cols), dtype=torch.float16, device=dev)
+        y = torch.empty((batch, rows), dtype=torch.float16, device=dev)
+        print_case("mm-long-row-time", batch)
+        assert capi.lowbit_gemm(q, s, x, y, cols, 128, bits) == 0
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            for _ in range(20):
+                assert capi.lowbit_gemm(q, s, x, y, cols, 128, bits) == 0
+        for _ in range(12):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            graph.replay()
+            a.record()
+            graph.replay()
+            b.record()
+            torch.cuda.synchronize()
+            best[batch] = min(best.get(batch, 1e9), a.elapsed_time(b))
+    assert best[1] < 0.93 * best[2], best
